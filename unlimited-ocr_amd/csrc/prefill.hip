@@ -104,10 +104,19 @@ void fwd_kernel(FwdK p) {
 
   // The hardware deals workgroups to the 8 XCDs round-robin; logical tile
   // xcd * per_xcd + k keeps neighbouring tiles of one (sequence, head), which
-  // share most of their window keys, on the same L2.
+  // share most of their window keys, on the same L2.  Paged: the requests'
+  // lengths differ and are known on the device only, so an eighth of the
+  // (request, head, tile) space is no eighth of the work; consecutive
+  // workgroups, on different XCDs, take one tile of each (request, head) in
+  // turn.  Six requests of 70 to 1,900 rows after 5k to 30k keys, ten heads:
+  // 236 -> 163 us; four of 2,048 rows, balanced either way: 145 -> 143 us
+  // (runs of 2, 4 and 8 tiles per XCD: 169 and 143 us).
   const int nwhole = p.nlogical - p.ntail;
   int lid, part = 0, rec = -1;
-  if ((int)blockIdx.x < 8 * p.per_xcd) {
+  if constexpr (PAGED) {
+    const int nbh = a.B * a.HQ;
+    lid = (int)blockIdx.x % nbh * p.ntiles + (int)blockIdx.x / nbh;
+  } else if ((int)blockIdx.x < 8 * p.per_xcd) {
     lid = (int)(blockIdx.x & 7) * p.per_xcd + (int)(blockIdx.x >> 3);
     if (lid >= nwhole) return;
   } else {
@@ -702,8 +711,8 @@ template <typename T, int D, bool PAGED, bool FP8 = false>
 int launch_fwd(const FwdK& k, size_t smem, hipStream_t st) {
   static LdsGrant granted;
   if (!ensure_dynamic_lds(&fwd_kernel<T, D, PAGED, FP8>, smem, &granted)) return SRSWA_UNSUPPORTED;
-  hipLaunchKernelGGL((fwd_kernel<T, D, PAGED, FP8>), dim3((unsigned)(8 * k.per_xcd + 8 * k.per_xcd_p)), dim3(128),
-                     smem, st, k);
+  const unsigned grid = PAGED ? (unsigned)k.nlogical : (unsigned)(8 * k.per_xcd + 8 * k.per_xcd_p);
+  hipLaunchKernelGGL((fwd_kernel<T, D, PAGED, FP8>), dim3(grid), dim3(128), smem, st, k);
   if constexpr (!PAGED)
     if (k.ntail > 0) hipLaunchKernelGGL((fwd_merge_kernel<T, D>), dim3((unsigned)(4 * k.ntail)), dim3(256), 0, st, k);
   const hipError_t e = hipGetLastError();
@@ -922,7 +931,6 @@ extern "C" int srswa_gather_fwd_paged(const srswa_paged_fwd_args* a, void* strea
     return SRSWA_UNSUPPORTED;
   }
   k.nlogical = (int)nlogical;
-  k.per_xcd = ceil_div(k.nlogical, 8);
   k.nsplit = 1;                    // no tail split: the live tiles depend on device-side lengths
   const int64_t per_tile = (int64_t)kTileRows * a->S * (ceil_div(a->page_size, kChunk) + 1) +
                            ceil_div(f.local_window + kTileRows - 1, kChunk) + 1;
