@@ -169,10 +169,11 @@ typedef struct {
 
 int srswa_gather_fwd(const srswa_fwd_args* a, void* stream);
 
-/* srswa_gather_fwd with a workspace for the tail split: when the launch's last
- * round of 64-row tiles would fill at most a fifth of the GPU, those tiles
- * run as four workgroups each over quarters of their key chunks, and a merge
- * kernel combines the parts (same masks, rounding points and outputs).  Bytes needed
+/* srswa_gather_fwd with a workspace for the split: when the launch's 64-row
+ * tiles fill at most half of the GPU, or the last of several rounds of them at
+ * most a fifth, those tiles run as 2, 4 or 8 workgroups each over parts of
+ * their key chunks, and a merge kernel combines the parts (same masks,
+ * rounding points and outputs).  Bytes needed
  * from srswa_gather_fwd_workspace (0: no split for this shape); ws NULL or
  * short runs every tile whole.  The same reference kernels as
  * srswa_gather_fwd (HF/sparse_gather_triton.py:35-122,
@@ -217,6 +218,16 @@ typedef struct {
 } srswa_paged_fwd_args;
 
 int srswa_gather_fwd_paged(const srswa_paged_fwd_args* a, void* stream);
+
+/* srswa_gather_fwd_paged with a workspace: a launch of few tiles runs each as
+ * several workgroups over parts of its key chunks, and a merge kernel combines
+ * the parts (same masks, rounding points and outputs).  Bytes needed from
+ * srswa_gather_fwd_paged_workspace (0: no split for this shape); ws NULL or
+ * short runs every tile whole.  The same reference kernel as
+ * srswa_gather_fwd_paged (WHL!layers/attention/unlimited_dash_ops/attend_triton.py:76-292);
+ * the split has no counterpart there. */
+size_t srswa_gather_fwd_paged_workspace(const srswa_paged_fwd_args* a);
+int srswa_gather_fwd_paged_ws(const srswa_paged_fwd_args* a, void* ws, size_t ws_bytes, void* stream);
 
 /* ------------------------------------------------------------------------
  * Gather-attention backward (dQ, dK, dV and the per-slot bias gradient).

@@ -108,3 +108,52 @@ def test_dash_sparse_attn_head_expanded_ids(dev):
     ref = O.paged_prefill_attend(q.double(), kc.double(), vc.double(), di.cpu().long(), db.cpu().double(),
                                  c["bt"].long(), c["cu"].tolist(), c["seq"].tolist(), c["ctx"].tolist(), 8, 0.088)
     assert_close_lowp(out.cpu(), ref, torch.bfloat16, 2e-2, "dash_sparse_attn head-expanded ids")
+
+
+@pytest.mark.parametrize("max_q,parts", [(64, 8), (190, 4), (640, 2), (1100, 1)])
+@pytest.mark.parametrize("kv", [None, torch.float8_e4m3fn])
+def test_split_launch_matches_whole_tiles(dev, monkeypatch, max_q, parts, kv):
+    """A launch of few tiles runs each as 8, 4 or 2 workgroups over parts of its
+    chunks (16 heads x 3 requests of ceil(max_q / 64) tiles, most of them past
+    their request's rows; a request of one key leaves parts without a chunk)
+    against every tile whole.  Each probability is rounded to bf16 (2^-9 of it)
+    relative to its part's own reference maximum, so the two forms round it
+    differently: they are at most 2 * 2^-9 * sum(p |v|) <= 2^-8 max|v| apart
+    before the output's own rounding (one unit in the last place)."""
+    import ctypes
+    from srswa import _lib
+    lib, H, D, page, K = _lib.lib(), 16, 128, 64, 8
+    g = torch.Generator().manual_seed(max_q)
+    q_lens, ctx = [max_q, 1, min(65, max_q)], [700, 0, 64 * 9 - 1]
+    seq = [a + b for a, b in zip(q_lens, ctx)]
+    nb = -(-max(seq) // page)
+    total = sum(q_lens)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)
+    q, kc, vc = rnd(total, H, D).to(dev), rnd(3 * nb, page, H, D), rnd(3 * nb, page, H, D)
+    kc, vc = (x.to(kv or torch.bfloat16).to(dev) for x in (kc, vc))
+    bt = torch.randperm(3 * nb, generator=g).view(3, nb).to(torch.int32).to(dev)
+    ids = torch.randint(-1, nb, (H, total, K), generator=g).to(torch.int32).to(dev)
+    bias = torch.randn(H, total, K, generator=g).to(dev)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)
+    cu = i32([0, q_lens[0], q_lens[0] + 1, total])
+    asked = []
+    real = lib.srswa_gather_fwd_paged_workspace
+
+    def run(split):
+        def workspace(a):
+            asked.append(real(a))
+            return asked[-1] if split else 0
+        monkeypatch.setattr(lib, "srswa_gather_fwd_paged_workspace", workspace)
+        out = torch.zeros(total, H, D, dtype=torch.bfloat16, device=dev)
+        U.dash_sparse_attn(q, kc, vc, ids, bias, bt, cu, i32(seq), i32(ctx), max_q, H, D ** -0.5, out, local_blocks=2,
+                           sparse_block_size=page)
+        return out.float()
+
+    whole, split = run(False), run(True)
+    tiles = 3 * H * -(-max_q // 64)
+    assert asked[0] == (0 if parts == 1 else tiles * parts * (64 * D + 128) * 4), (asked, tiles)
+    assert torch.isfinite(split).all()
+    ulp = torch.exp2(torch.floor(torch.log2(whole.abs().clamp(min=1e-3))) - 7)
+    assert ((split - whole).abs() <= 2.0 ** -8 * vc.float().abs().max() + ulp).all()
+    if parts == 1:
+        assert torch.equal(split, whole)

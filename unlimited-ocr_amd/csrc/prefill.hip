@@ -115,7 +115,12 @@ void fwd_kernel(FwdK p) {
   int lid, part = 0, rec = -1;
   if constexpr (PAGED) {
     const int nbh = a.B * a.HQ;
-    lid = (int)blockIdx.x % nbh * p.ntiles + (int)blockIdx.x / nbh;
+    const int ti = (int)blockIdx.x / p.nsplit;
+    lid = ti % nbh * p.ntiles + ti / nbh;
+    if (p.nsplit > 1) {
+      part = (int)blockIdx.x % p.nsplit;
+      rec = lid * p.nsplit + part;
+    }
   } else if ((int)blockIdx.x < 8 * p.per_xcd) {
     lid = (int)(blockIdx.x & 7) * p.per_xcd + (int)(blockIdx.x >> 3);
     if (lid >= nwhole) return;
@@ -586,13 +591,13 @@ void fwd_kernel(FwdK p) {
         l_tot > 0.f ? (m_b + log2f(l_tot)) * kLn2 : -INFINITY;
 }
 
-// Combines the nsplit (<= 4) part records of each split tile: m = max m_p,
+// Combines the NS (2, 4 or 8) part records of each split tile: m = max m_p,
 // O = sum 2^(m_p - m) O_p, l = sum 2^(m_p - m) l_p, out = O / l in the input
 // dtype, lse = (m + log2 l) ln 2.  A row with no keys in any part (l = 0)
 // writes zeros and lse = -inf, as the unsplit kernel does.  Four workgroups
 // per tile (16 rows each), 16 threads per row, every part's loads issued
 // before the combine.
-template <typename T, int D>
+template <typename T, int D, bool PAGED, int NS>
 __global__ __launch_bounds__(256) void fwd_merge_kernel(FwdK p) {
   using M = Mfma<T>;
   constexpr int TPR = 16, DPT = D / TPR;         // threads per row, dims per thread (8 or 4)
@@ -603,27 +608,32 @@ __global__ __launch_bounds__(256) void fwd_merge_kernel(FwdK p) {
   const int tile = lid % p.ntiles, bh = lid / p.ntiles;
   const int hq = bh % a.HQ, b = bh / a.HQ;
   const int t0 = tile * kTileRows;
-  const int nrows = min(kTileRows, a.T - t0);
+  int q0 = 0, Tb = a.T;
+  if constexpr (PAGED) {
+    q0 = p.cu[b];
+    Tb = p.cu[b + 1] - q0;
+  }
+  const int nrows = min(kTileRows, Tb - t0);      // none: a tile past its request's rows
   const int r = 16 * ((int)blockIdx.x & 3) + (int)threadIdx.x / TPR, c = (int)threadIdx.x % TPR;
   if (r >= nrows) return;
-  const float* rec = p.part + (int64_t)ti * p.nsplit * REC;
-  float2 ml[4];
-  float4 ov[4][DPT / 4];
+  const float* rec = p.part + (int64_t)ti * NS * REC;
+  float2 ml[NS];
+  float4 ov[NS][DPT / 4];
+  float mx = -INFINITY;
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const bool live = q < p.nsplit;
-    const float* pq = rec + (int64_t)(live ? q : 0) * REC;
-    ml[q] = live ? *reinterpret_cast<const float2*>(pq + 64 * D + 2 * r) : make_float2(-INFINITY, 0.f);
+  for (int q = 0; q < NS; ++q) {
+    const float* pq = rec + (int64_t)q * REC;
+    ml[q] = *reinterpret_cast<const float2*>(pq + 64 * D + 2 * r);
 #pragma unroll
-    for (int d = 0; d < DPT / 4; ++d)
-      ov[q][d] = live ? reinterpret_cast<const float4*>(pq + r * D + c * DPT)[d] : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int d = 0; d < DPT / 4; ++d) ov[q][d] = reinterpret_cast<const float4*>(pq + r * D + c * DPT)[d];
   }
-  const float mx = fmaxf(fmaxf(ml[0].x, ml[1].x), fmaxf(ml[2].x, ml[3].x));
+#pragma unroll
+  for (int q = 0; q < NS; ++q) mx = fmaxf(mx, ml[q].x);
   float l = 0.f, acc[DPT];
 #pragma unroll
   for (int d = 0; d < DPT; ++d) acc[d] = 0.f;
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
+  for (int q = 0; q < NS; ++q) {
     const float w = ml[q].x == -INFINITY ? 0.f : exp2f(ml[q].x - mx);
     l += ml[q].y * w;
 #pragma unroll
@@ -635,8 +645,8 @@ __global__ __launch_bounds__(256) void fwd_merge_kernel(FwdK p) {
     }
   }
   const float inv = l > 0.f ? 1.f / l : 0.f;
-  T* orow = reinterpret_cast<T*>(a.out) + (int64_t)b * a.o_sb + (int64_t)(t0 + r) * a.o_st + (int64_t)hq * a.o_sh +
-            c * DPT;
+  T* orow = reinterpret_cast<T*>(a.out) + (int64_t)b * a.o_sb + (int64_t)(q0 + t0 + r) * a.o_st +
+            (int64_t)hq * a.o_sh + c * DPT;
   if constexpr (std::is_same<T, float>::value) {
 #pragma unroll
     for (int d = 0; d < DPT / 4; ++d)
@@ -649,7 +659,7 @@ __global__ __launch_bounds__(256) void fwd_merge_kernel(FwdK p) {
   } else {
     *reinterpret_cast<uint2*>(orow) = make_uint2(M::pack2(acc[0] * inv, acc[1] * inv), M::pack2(acc[2] * inv, acc[3] * inv));
   }
-  if (c == 0 && a.lse)
+  if (!PAGED && c == 0 && a.lse)
     a.lse[(int64_t)b * a.lse_sb + (int64_t)(t0 + r) * a.lse_st + (int64_t)hq * a.lse_sh] =
         l > 0.f ? (mx + log2f(l)) * kLn2 : -INFINITY;
 }
@@ -711,10 +721,14 @@ template <typename T, int D, bool PAGED, bool FP8 = false>
 int launch_fwd(const FwdK& k, size_t smem, hipStream_t st) {
   static LdsGrant granted;
   if (!ensure_dynamic_lds(&fwd_kernel<T, D, PAGED, FP8>, smem, &granted)) return SRSWA_UNSUPPORTED;
-  const unsigned grid = PAGED ? (unsigned)k.nlogical : (unsigned)(8 * k.per_xcd + 8 * k.per_xcd_p);
+  const unsigned grid = PAGED ? (unsigned)(k.nlogical * k.nsplit) : (unsigned)(8 * k.per_xcd + 8 * k.per_xcd_p);
   hipLaunchKernelGGL((fwd_kernel<T, D, PAGED, FP8>), dim3(grid), dim3(128), smem, st, k);
-  if constexpr (!PAGED)
-    if (k.ntail > 0) hipLaunchKernelGGL((fwd_merge_kernel<T, D>), dim3((unsigned)(4 * k.ntail)), dim3(256), 0, st, k);
+  if (k.ntail > 0) {
+    const dim3 mg((unsigned)(4 * k.ntail));
+    if (k.nsplit == 8) hipLaunchKernelGGL((fwd_merge_kernel<T, D, PAGED, 8>), mg, dim3(256), 0, st, k);
+    else if (k.nsplit == 4) hipLaunchKernelGGL((fwd_merge_kernel<T, D, PAGED, 4>), mg, dim3(256), 0, st, k);
+    else hipLaunchKernelGGL((fwd_merge_kernel<T, D, PAGED, 2>), mg, dim3(256), 0, st, k);
+  }
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
     set_error("fwd launch failed: %s", hipGetErrorString(e));
@@ -730,6 +744,19 @@ using namespace srswa;
 
 namespace srswa {
 namespace {
+
+// Parts per tile of a round of `tiles` tiles on a GPU that holds `slots`
+// workgroups.  A launch of one round (`alone`) takes as many of 8, 4 or 2 as
+// the slots hold: a tile's chunks are a chain of load latencies, and idle CUs
+// run the parts at once.  One request behind 30,000 keys, ten heads, biased
+// rows of their own selections (17 to 21 chunks a tile), whole -> split: 40
+// tiles 70 -> 28 us (8 parts), 120 tiles 71 -> 41 (4), 190 tiles 71 -> 46 (4),
+// 250 tiles 71 -> 58 (2), 380 tiles 86 -> 67 (2).  The last round of several
+// only up to a fifth of the slots, in 4 parts: see below.
+int split_parts(int64_t tiles, int64_t slots, bool alone) {
+  if (!alone) return tiles * 5 <= slots ? 4 : 1;
+  return tiles * 8 <= slots ? 8 : tiles * 4 <= slots ? 4 : tiles * 2 <= slots ? 2 : 1;
+}
 
 // The forward's launch plan (no device work).  Returns SRSWA_OK with k, smem
 // and the split's workspace bytes filled in.
@@ -768,16 +795,15 @@ int plan_fwd(const srswa_fwd_args* a, FwdK& k, size_t& smem, size_t& ws_bytes) {
     set_error("fwd: %zu bytes of LDS needed (key length too large)", smem);
     return SRSWA_UNSUPPORTED;
   }
-  // Tail split.  The GPU holds `slots` workgroups at once (four per CU at two
-  // waves per SIMD, fewer when LDS runs out).  When the last round of tiles
-  // fills at most a fifth of them, its tiles run as four workgroups each over
-  // quarters of their chunk plans, so that round takes about a quarter of a
-  // tile's time.  A fuller last round is left whole: each part pays the
-  // tile's set-up and first-load latency again, and its fp32 record costs
-  // 8x the tile's output bytes, which outweighs the shorter round.  Measured
-  // (4 x 10 heads, 65536 keys, D 128): 80 tiles 39.5 -> 27.6 us, 200 tiles
-  // 40.9 -> 38.6 us, 1,040 tiles 110 -> 92 us split; 1,280 tiles on 1,024
-  // slots 129 us whole against 134 us split.
+  // Split of the last round.  The GPU holds `slots` workgroups at once (four
+  // per CU at two waves per SIMD, fewer when LDS runs out).  When the last
+  // round of several fills at most a fifth of them, its tiles run as four
+  // workgroups each over quarters of their chunk plans, so that round takes
+  // about a quarter of a tile's time.  A fuller last round is left whole: each
+  // part pays the tile's set-up and first-load latency again, and its fp32
+  // record costs 8x the tile's output bytes, which outweighs the shorter
+  // round.  Measured (4 x 10 heads, 65536 keys, D 128): 1,040 tiles 110 -> 92
+  // us split; 1,280 tiles on 1,024 slots 125 us whole against 132 us split.
   k.nsplit = 1;
   k.ntail = 0;
   ws_bytes = 0;
@@ -787,11 +813,10 @@ int plan_fwd(const srswa_fwd_args* a, FwdK& k, size_t& smem, size_t& ws_bytes) {
     const int64_t slots = (int64_t)cus * per_cu;
     const int64_t rounds = (nlogical + slots - 1) / slots;
     const int64_t tail = nlogical - (rounds - 1) * slots;
-    const int64_t f = 4;
-    if (tail * 5 <= slots) {
-      k.nsplit = (int)f;
+    k.nsplit = split_parts(tail, slots, rounds == 1);
+    if (k.nsplit > 1) {
       k.ntail = (int)tail;
-      ws_bytes = (size_t)tail * f * (64 * a->D + 128) * sizeof(float);
+      ws_bytes = (size_t)tail * k.nsplit * (64 * a->D + 128) * sizeof(float);
     }
   }
   k.per_xcd = ceil_div(k.nlogical - k.ntail, 8);
@@ -837,7 +862,13 @@ extern "C" int srswa_gather_fwd(const srswa_fwd_args* a, void* stream) {
   return srswa_gather_fwd_ws(a, nullptr, 0, stream);
 }
 
-extern "C" int srswa_gather_fwd_paged(const srswa_paged_fwd_args* a, void* stream) {
+namespace srswa {
+namespace {
+
+// The paged form's launch plan, as plan_fwd
+int plan_fwd_paged(const srswa_paged_fwd_args* a, FwdK& k, size_t& smem, size_t& ws_bytes) {
+  ws_bytes = 0;
+  k = FwdK{};
   if (!a || !a->q || !a->k_cache || !a->v_cache || !a->out || !a->block_table || !a->cu_seqlens_q ||
       !a->seq_lens || !a->prefix_lens || (!a->topk && a->S > 0)) {
     set_error("paged fwd: null argument");
@@ -848,7 +879,7 @@ extern "C" int srswa_gather_fwd_paged(const srswa_paged_fwd_args* a, void* strea
     set_error("paged fwd: bad sizes");
     return SRSWA_INVALID;
   }
-  if (a->R == 0 || a->max_query_len == 0) return SRSWA_OK;
+  if (a->R == 0 || a->max_query_len == 0) return SRSWA_OK;   // nothing to launch (nlogical 0)
   if (a->HQ % a->HKV) {
     set_error("paged fwd: HQ must be a multiple of HKV");
     return SRSWA_UNSUPPORTED;
@@ -897,7 +928,6 @@ extern "C" int srswa_gather_fwd_paged(const srswa_paged_fwd_args* a, void* strea
     set_error("paged fwd: pointers must be 16-byte aligned");
     return SRSWA_UNSUPPORTED;
   }
-  FwdK k{};
   srswa_fwd_args& f = k.a;
   f.q = a->q;  f.q_sb = 0;  f.q_st = a->q_sn;  f.q_sh = a->q_sh;
   f.k = a->k_cache;  f.k_sb = 0;  f.k_st = a->k_st;  f.k_sh = a->k_sh;
@@ -931,7 +961,6 @@ extern "C" int srswa_gather_fwd_paged(const srswa_paged_fwd_args* a, void* strea
     return SRSWA_UNSUPPORTED;
   }
   k.nlogical = (int)nlogical;
-  k.nsplit = 1;                    // no tail split: the live tiles depend on device-side lengths
   const int64_t per_tile = (int64_t)kTileRows * a->S * (ceil_div(a->page_size, kChunk) + 1) +
                            ceil_div(f.local_window + kTileRows - 1, kChunk) + 1;
   const int umax = (int)std::min<int64_t>(nchunk, per_tile);
@@ -949,11 +978,44 @@ extern "C" int srswa_gather_fwd_paged(const srswa_paged_fwd_args* a, void* strea
   const size_t budget = k.pages_off <= 40 * 1024 - 64 ? 40 * 1024 : 52 * 1024;
   k.page_cap = (int)std::min<int64_t>(umax, k.pages_off < (int)budget ? (budget - k.pages_off) / (4 * k.ppc) : 0);
   n = k.pages_off + (size_t)k.page_cap * 4 * k.ppc;
-  const size_t smem = (n + 15) / 16 * 16;
+  smem = (n + 15) / 16 * 16;
   if (smem > 156 * 1024) {
     set_error("paged fwd: %zu bytes of LDS needed (block table too wide)", smem);
     return SRSWA_UNSUPPORTED;
   }
+  // every tile is split or none: which tiles are live is known on the device only
+  k.nsplit = 1;
+  const int cus = device_cu_count();
+  const int per_cu = std::min<int>(4, (int)((160 * 1024) / smem));
+  if (cus > 0 && per_cu > 0) k.nsplit = split_parts(nlogical, (int64_t)cus * per_cu, true);
+  if (k.nsplit > 1) {
+    k.ntail = k.nlogical;
+    ws_bytes = (size_t)nlogical * k.nsplit * (64 * a->D + 128) * sizeof(float);
+  }
+  return SRSWA_OK;
+}
+
+}  // namespace
+}  // namespace srswa
+
+extern "C" size_t srswa_gather_fwd_paged_workspace(const srswa_paged_fwd_args* a) {
+  FwdK k;
+  size_t smem = 0, ws = 0;
+  return plan_fwd_paged(a, k, smem, ws) == SRSWA_OK ? ws : 0;
+}
+
+extern "C" int srswa_gather_fwd_paged_ws(const srswa_paged_fwd_args* a, void* ws, size_t ws_bytes, void* stream) {
+  FwdK k;
+  size_t smem = 0, need = 0;
+  const int st = plan_fwd_paged(a, k, smem, need);
+  if (st != SRSWA_OK || k.nlogical == 0) return st;
+  if (k.ntail > 0 && (!ws || ws_bytes < need || ((uintptr_t)ws & 15u))) {
+    // no (usable) workspace: every tile runs whole
+    k.nsplit = 1;
+    k.ntail = 0;
+  }
+  k.part = reinterpret_cast<float*>(ws);
+  const bool fp8 = a->kv_fp8 != 0;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (fp8) {
     if (a->dtype == SRSWA_BF16)
@@ -964,4 +1026,8 @@ extern "C" int srswa_gather_fwd_paged(const srswa_paged_fwd_args* a, void* strea
   if (a->dtype == SRSWA_BF16)
     return a->D == 128 ? launch_fwd<bf16_t, 128, true>(k, smem, s) : launch_fwd<bf16_t, 64, true>(k, smem, s);
   return a->D == 128 ? launch_fwd<__half, 128, true>(k, smem, s) : launch_fwd<__half, 64, true>(k, smem, s);
+}
+
+extern "C" int srswa_gather_fwd_paged(const srswa_paged_fwd_args* a, void* stream) {
+  return srswa_gather_fwd_paged_ws(a, nullptr, 0, stream);
 }

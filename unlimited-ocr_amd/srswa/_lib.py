@@ -574,6 +574,8 @@ SIGNATURES = {
     "srswa_gather_fwd_workspace": (ctypes.c_size_t, [ctypes.POINTER(FwdArgs)]),
     "srswa_gather_fwd_ws": (ctypes.c_int, [ctypes.POINTER(FwdArgs), _vp, ctypes.c_size_t, _vp]),
     "srswa_gather_fwd_paged": (ctypes.c_int, [ctypes.POINTER(PagedFwdArgs), _vp]),
+    "srswa_gather_fwd_paged_workspace": (ctypes.c_size_t, [ctypes.POINTER(PagedFwdArgs)]),
+    "srswa_gather_fwd_paged_ws": (ctypes.c_int, [ctypes.POINTER(PagedFwdArgs), _vp, ctypes.c_size_t, _vp]),
     "srswa_gather_bwd_workspace": (ctypes.c_size_t, [ctypes.POINTER(BwdArgs)]),
     "srswa_gather_bwd": (ctypes.c_int, [ctypes.POINTER(BwdArgs), _vp, ctypes.c_size_t, _vp]),
     "srswa_block_max_score": (ctypes.c_int, [ctypes.POINTER(BlockMaxArgs), _vp]),

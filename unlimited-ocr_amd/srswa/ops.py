@@ -413,8 +413,11 @@ def gather_fwd_paged(q, k_cache, v_cache, topk_idx, blk_bias, block_table, cu_se
     a.scale = float(scale)
     a.dtype = _lib.dtype_code(q.dtype)
     a.kv_fp8 = kv8
-    _lib.check(_lib.lib().srswa_gather_fwd_paged(ctypes.byref(a), _lib.stream_ptr(q.device)),
-               "srswa_gather_fwd_paged")
+    # the split's workspace (0 bytes for a launch that fills the GPU)
+    nws = _lib.lib().srswa_gather_fwd_paged_workspace(ctypes.byref(a))
+    ws = torch.empty(nws, dtype=torch.uint8, device=q.device) if nws else None
+    _lib.check(_lib.lib().srswa_gather_fwd_paged_ws(ctypes.byref(a), _lib.ptr(ws), nws, _lib.stream_ptr(q.device)),
+               "srswa_gather_fwd_paged_ws")
     return out
 
 
