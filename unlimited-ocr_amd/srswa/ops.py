@@ -26,6 +26,13 @@ def _i32(t: torch.Tensor) -> torch.Tensor:
     return t if t.dtype == torch.int32 else t.to(torch.int32)
 
 
+def _as(t: torch.Tensor, dtype: torch.dtype, shape) -> torch.Tensor:
+    """``t`` in ``dtype``, broadcast to ``shape`` and dense (itself when it is all three)."""
+    if t.dtype != dtype:
+        t = t.to(dtype)
+    return (t if t.shape == shape else t.expand(shape)).contiguous()
+
+
 class _Launch:
     """A prepared launch: the C-ABI struct, the tensors it points into (kept
     alive), the scratch buffer and the entry point.  ``__call__``
@@ -74,9 +81,9 @@ def prepare_gather_decode(q, k_cache, v_cache, block_indices, q_pos, *, block_si
             raise UnsupportedShape("head dim must be contiguous")
     idx = _i32(block_indices).contiguous()
     if bias is not None:
-        bias = bias.to(torch.float32).expand(idx.shape).contiguous()
+        bias = _as(bias, torch.float32, idx.shape)
     if valid is not None:
-        valid = valid.to(torch.bool).expand(idx.shape).contiguous().view(torch.uint8)
+        valid = _as(valid, torch.bool, idx.shape).view(torch.uint8)
     pos = _i32(q_pos).contiguous()
     if tuple(pos.shape) != (B, Lq):
         raise ValueError(f"q_pos shape {tuple(pos.shape)} != {(B, Lq)}")
@@ -89,18 +96,18 @@ def prepare_gather_decode(q, k_cache, v_cache, block_indices, q_pos, *, block_si
     lse = torch.empty(B, Lq, HQ, dtype=torch.float32, device=q.device) if return_lse else None
 
     a = _lib.DecodeArgs()
-    a.q = q.data_ptr(); a.q_sb, a.q_sq, a.q_sh = q.stride(0), q.stride(1), q.stride(2)
-    a.k = k_cache.data_ptr(); a.k_sb, a.k_st, a.k_sh = k_cache.stride(0), k_cache.stride(1), k_cache.stride(2)
-    a.v = v_cache.data_ptr(); a.v_sb, a.v_st, a.v_sh = v_cache.stride(0), v_cache.stride(1), v_cache.stride(2)
+    a.q = q.data_ptr(); a.q_sb, a.q_sq, a.q_sh = q.stride()[:3]
+    a.k = k_cache.data_ptr(); a.k_sb, a.k_st, a.k_sh = k_cache.stride()[:3]
+    a.v = v_cache.data_ptr(); a.v_sb, a.v_st, a.v_sh = v_cache.stride()[:3]
     a.idx = idx.data_ptr()
-    a.idx_sb, a.idx_sh, a.idx_sq, a.idx_ss = idx.stride(0), idx.stride(1), idx.stride(2), idx.stride(3)
+    a.idx_sb, a.idx_sh, a.idx_sq, a.idx_ss = idx.stride()[:4]
     a.bias = _lib.ptr(bias)
     a.valid = _lib.ptr(valid)
-    a.q_pos = pos.data_ptr(); a.pos_sb, a.pos_sq = pos.stride(0), pos.stride(1)
+    a.q_pos = pos.data_ptr(); a.pos_sb, a.pos_sq = pos.stride()[:2]
     a.kv_len = _lib.ptr(kvl)
-    a.out = out.data_ptr(); a.o_sb, a.o_sq, a.o_sh = out.stride(0), out.stride(1), out.stride(2)
+    a.out = out.data_ptr(); a.o_sb, a.o_sq, a.o_sh = out.stride()[:3]
     if lse is not None:
-        a.lse = lse.data_ptr(); a.lse_sb, a.lse_sq, a.lse_sh = lse.stride(0), lse.stride(1), lse.stride(2)
+        a.lse = lse.data_ptr(); a.lse_sb, a.lse_sq, a.lse_sh = lse.stride()[:3]
     a.B, a.Lq, a.HQ, a.HKV, a.HI, a.D, a.S, a.L = B, Lq, HQ, HKV, HI, D, S, L
     a.block_size, a.local_window = int(block_size), max(1, int(local_window))
     a.scale = float(scale)
@@ -197,18 +204,18 @@ def prepare_index_meanpool_topk(q, k, q_pos, *, block_size, local_blocks, topk, 
     idx = torch.empty(B, HI, Lq, int(topk), dtype=torch.int32, device=q.device) if topk > 0 else None
 
     a = _lib.IndexArgs()
-    a.q = qf.data_ptr(); a.q_sb, a.q_sh, a.q_sq = qf.stride(0), qf.stride(1), qf.stride(2)
-    a.k = k.data_ptr(); a.k_sb, a.k_st = k.stride(0), k.stride(1)
+    a.q = qf.data_ptr(); a.q_sb, a.q_sh, a.q_sq = qf.stride()[:3]
+    a.k = k.data_ptr(); a.k_sb, a.k_st = k.stride()[:2]
     a.k_sh = 0 if HK == 1 else k.stride(2)
     if kbar is not None:
-        a.kbar_out = kbar.data_ptr(); a.kb_sb, a.kb_sh, a.kb_sn = kbar.stride(0), kbar.stride(1), kbar.stride(2)
+        a.kbar_out = kbar.data_ptr(); a.kb_sb, a.kb_sh, a.kb_sn = kbar.stride()[:3]
     a.head_cls = _lib.ptr(hc)
-    a.q_pos = pos.data_ptr(); a.pos_sb, a.pos_sq = pos.stride(0), pos.stride(1)
+    a.q_pos = pos.data_ptr(); a.pos_sb, a.pos_sq = pos.stride()[:2]
     a.kv_len = _lib.ptr(kvl)
     if scores is not None:
-        a.scores = scores.data_ptr(); a.sc_sb, a.sc_sh, a.sc_sq = scores.stride(0), scores.stride(1), scores.stride(2)
+        a.scores = scores.data_ptr(); a.sc_sb, a.sc_sh, a.sc_sq = scores.stride()[:3]
     if idx is not None:
-        a.topk_idx = idx.data_ptr(); a.ti_sb, a.ti_sh, a.ti_sq = idx.stride(0), idx.stride(1), idx.stride(2)
+        a.topk_idx = idx.data_ptr(); a.ti_sb, a.ti_sh, a.ti_sq = idx.stride()[:3]
     a.B, a.HI, a.Lq, a.D, a.L, a.nblk = B, HI, Lq, D, L, nblk
     a.block_size, a.local_blocks, a.K, a.ascending = int(block_size), int(local_blocks), int(topk), int(bool(ascending))
     a.k_dtype = _lib.dtype_code(k.dtype)
@@ -324,14 +331,14 @@ def prepare_gather_decode_paged(q, k_cache, v_cache, topk_idx, blk_bias, block_t
     if out is None:
         out = torch.empty(total_q, HQ, D, dtype=q.dtype, device=q.device)
     a = _lib.PagedDecodeArgs()
-    a.q = q.data_ptr(); a.q_sn, a.q_sh = q.stride(0), q.stride(1)
-    a.k_cache = k_cache.data_ptr(); a.k_sp, a.k_st, a.k_sh = k_cache.stride(0), k_cache.stride(1), k_cache.stride(2)
-    a.v_cache = v_cache.data_ptr(); a.v_sp, a.v_st, a.v_sh = v_cache.stride(0), v_cache.stride(1), v_cache.stride(2)
-    a.topk = ti.data_ptr(); a.t_sh, a.t_sn, a.t_sk = ti.stride(0), ti.stride(1), ti.stride(2)
+    a.q = q.data_ptr(); a.q_sn, a.q_sh = q.stride()[:2]
+    a.k_cache = k_cache.data_ptr(); a.k_sp, a.k_st, a.k_sh = k_cache.stride()[:3]
+    a.v_cache = v_cache.data_ptr(); a.v_sp, a.v_st, a.v_sh = v_cache.stride()[:3]
+    a.topk = ti.data_ptr(); a.t_sh, a.t_sn, a.t_sk = ti.stride()[:3]
     a.bias = _lib.ptr(bias)
     a.block_table = bt.data_ptr(); a.bt_sr = bt.stride(0)
     a.seq_lens = sl.data_ptr()
-    a.out = out.data_ptr(); a.o_sn, a.o_sh = out.stride(0), out.stride(1)
+    a.out = out.data_ptr(); a.o_sn, a.o_sh = out.stride()[:2]
     a.R, a.dql, a.HQ, a.HKV, a.D, a.topk_n = R, dql, HQ, HKV, D, ti.shape[-1]
     a.max_blocks, a.page_size, a.local_blocks = bt.shape[1], page, int(local_blocks)
     a.scale = float(scale)
@@ -399,15 +406,15 @@ def gather_fwd_paged(q, k_cache, v_cache, topk_idx, blk_bias, block_table, cu_se
     if out is None:
         out = torch.empty(total_q, HQ, D, dtype=q.dtype, device=q.device)
     a = _lib.PagedFwdArgs()
-    a.q = q.data_ptr(); a.q_sn, a.q_sh = q.stride(0), q.stride(1)
-    a.k_cache = k_cache.data_ptr(); a.k_sp, a.k_st, a.k_sh = k_cache.stride(0), k_cache.stride(1), k_cache.stride(2)
-    a.v_cache = v_cache.data_ptr(); a.v_sp, a.v_st, a.v_sh = v_cache.stride(0), v_cache.stride(1), v_cache.stride(2)
-    a.topk = ti.data_ptr(); a.t_sh, a.t_sn = ti.stride(0), ti.stride(1)
+    a.q = q.data_ptr(); a.q_sn, a.q_sh = q.stride()[:2]
+    a.k_cache = k_cache.data_ptr(); a.k_sp, a.k_st, a.k_sh = k_cache.stride()[:3]
+    a.v_cache = v_cache.data_ptr(); a.v_sp, a.v_st, a.v_sh = v_cache.stride()[:3]
+    a.topk = ti.data_ptr(); a.t_sh, a.t_sn = ti.stride()[:2]
     if bias is not None:
-        a.bias = bias.data_ptr(); a.b_sh, a.b_sn = bias.stride(0), bias.stride(1)
+        a.bias = bias.data_ptr(); a.b_sh, a.b_sn = bias.stride()[:2]
     a.block_table = bt.data_ptr(); a.bt_sr = bt.stride(0)
     a.cu_seqlens_q, a.seq_lens, a.prefix_lens = cu.data_ptr(), sl.data_ptr(), pl.data_ptr()
-    a.out = out.data_ptr(); a.o_sn, a.o_sh = out.stride(0), out.stride(1)
+    a.out = out.data_ptr(); a.o_sn, a.o_sh = out.stride()[:2]
     a.R, a.max_query_len, a.HQ, a.HKV, a.D, a.S = R, int(max_query_len), HQ, HKV, D, ti.shape[-1]
     a.max_blocks, a.page_size, a.local_blocks = bt.shape[1], page, int(local_blocks)
     a.scale = float(scale)
@@ -614,8 +621,8 @@ def _seg_from_positions(position_ids, T, Sk, device):
     if position_ids is None:
         return None
     qi = torch.arange(Sk - T, Sk, device=device, dtype=torch.int64)
-    seg = (qi[None, :] - position_ids.to(device=device, dtype=torch.int64)).to(torch.int32).contiguous()
-    return seg
+    pos = position_ids.to(device=device, dtype=torch.int64)
+    return torch.sub(qi, pos, out=torch.empty(pos.shape, dtype=torch.int32, device=device))   # narrowed as it is stored
 
 
 def gather_fwd(q, k, v, block_indices, *, block_size, local_window, scale, seg=None, bias=None,
@@ -644,24 +651,24 @@ def gather_fwd(q, k, v, block_indices, *, block_size, local_window, scale, seg=N
     if bias is not None:
         if bias.dim() == 3:
             bias = bias.unsqueeze(1)
-        bias = bias.to(torch.float32).expand(B, HI, T, S).contiguous()
+        bias = _as(bias, torch.float32, idx.shape)
     if seg is not None:
         seg = _i32(seg).contiguous()
     if out is None:
         out = torch.empty(B, T, HQ, D, dtype=q.dtype, device=q.device)
     lse = torch.empty(B, T, HQ, dtype=torch.float32, device=q.device) if need_lse else None
     a = _lib.FwdArgs()
-    a.q = q.data_ptr(); a.q_sb, a.q_st, a.q_sh = q.stride(0), q.stride(1), q.stride(2)
-    a.k = k.data_ptr(); a.k_sb, a.k_st, a.k_sh = k.stride(0), k.stride(1), k.stride(2)
-    a.v = v.data_ptr(); a.v_sb, a.v_st, a.v_sh = v.stride(0), v.stride(1), v.stride(2)
-    a.idx = idx.data_ptr(); a.idx_sb, a.idx_sh, a.idx_st = idx.stride(0), idx.stride(1), idx.stride(2)
+    a.q = q.data_ptr(); a.q_sb, a.q_st, a.q_sh = q.stride()[:3]
+    a.k = k.data_ptr(); a.k_sb, a.k_st, a.k_sh = k.stride()[:3]
+    a.v = v.data_ptr(); a.v_sb, a.v_st, a.v_sh = v.stride()[:3]
+    a.idx = idx.data_ptr(); a.idx_sb, a.idx_sh, a.idx_st = idx.stride()[:3]
     if bias is not None:
-        a.bias = bias.data_ptr(); a.bias_sb, a.bias_sh, a.bias_st = bias.stride(0), bias.stride(1), bias.stride(2)
+        a.bias = bias.data_ptr(); a.bias_sb, a.bias_sh, a.bias_st = bias.stride()[:3]
     if seg is not None:
         a.seg = seg.data_ptr(); a.seg_sb = seg.stride(0)
-    a.out = out.data_ptr(); a.o_sb, a.o_st, a.o_sh = out.stride(0), out.stride(1), out.stride(2)
+    a.out = out.data_ptr(); a.o_sb, a.o_st, a.o_sh = out.stride()[:3]
     if lse is not None:
-        a.lse = lse.data_ptr(); a.lse_sb, a.lse_st, a.lse_sh = lse.stride(0), lse.stride(1), lse.stride(2)
+        a.lse = lse.data_ptr(); a.lse_sb, a.lse_st, a.lse_sh = lse.stride()[:3]
     a.B, a.T, a.Sk, a.HQ, a.HKV, a.HI, a.D, a.S = B, T, Sk, HQ, HKV, HI, D, S
     a.block_size, a.local_window = int(block_size), max(1, int(local_window))
     a.scale = float(scale)
@@ -687,7 +694,7 @@ def gather_bwd(q, k, v, o, lse, do, block_indices, *, block_size, local_window, 
     if bias is not None:
         if bias.dim() == 3:
             bias = bias.unsqueeze(1)
-        bias = bias.to(torch.float32).expand(B, HI, T, S).contiguous()
+        bias = _as(bias, torch.float32, idx.shape)
     if seg is not None:
         seg = _i32(seg).contiguous()
     if do.stride(-1) != 1:
@@ -700,19 +707,20 @@ def gather_bwd(q, k, v, o, lse, do, block_indices, *, block_size, local_window, 
         dbh = torch.empty(B, HQ, T, S, dtype=torch.float32, device=q.device)
     a = _lib.BwdArgs()
     for name, t in (("q", q), ("k", k), ("v", v), ("o", o), ("dq", dq), ("dk", dk), ("dv", dv)):
+        st = t.stride()
         setattr(a, name, t.data_ptr())
-        setattr(a, name + "_sb", t.stride(0))
-        setattr(a, name + "_st", t.stride(1))
-        setattr(a, name + "_sh", t.stride(2))
-    a.dout = do.data_ptr(); a.do_sb, a.do_st, a.do_sh = do.stride(0), do.stride(1), do.stride(2)
-    a.lse = lse.data_ptr(); a.lse_sb, a.lse_st, a.lse_sh = lse.stride(0), lse.stride(1), lse.stride(2)
-    a.idx = idx.data_ptr(); a.idx_sb, a.idx_sh, a.idx_st = idx.stride(0), idx.stride(1), idx.stride(2)
+        setattr(a, name + "_sb", st[0])
+        setattr(a, name + "_st", st[1])
+        setattr(a, name + "_sh", st[2])
+    a.dout = do.data_ptr(); a.do_sb, a.do_st, a.do_sh = do.stride()[:3]
+    a.lse = lse.data_ptr(); a.lse_sb, a.lse_st, a.lse_sh = lse.stride()[:3]
+    a.idx = idx.data_ptr(); a.idx_sb, a.idx_sh, a.idx_st = idx.stride()[:3]
     if bias is not None:
-        a.bias = bias.data_ptr(); a.bias_sb, a.bias_sh, a.bias_st = bias.stride(0), bias.stride(1), bias.stride(2)
+        a.bias = bias.data_ptr(); a.bias_sb, a.bias_sh, a.bias_st = bias.stride()[:3]
     if seg is not None:
         a.seg = seg.data_ptr(); a.seg_sb = seg.stride(0)
     if dbh is not None:
-        a.dbias = dbh.data_ptr(); a.db_sb, a.db_sh, a.db_st = dbh.stride(0), dbh.stride(1), dbh.stride(2)
+        a.dbias = dbh.data_ptr(); a.db_sb, a.db_sh, a.db_st = dbh.stride()[:3]
     a.B, a.T, a.Sk, a.HQ, a.HKV, a.HI, a.D, a.S = B, T, Sk, HQ, HKV, HI, D, S
     a.block_size, a.local_window = int(block_size), max(1, int(local_window))
     a.scale = float(scale)
@@ -776,12 +784,12 @@ def block_max_score(q, k, pos, seg, *, block_size, num_key_blocks, local_window)
     segi = None if seg is None else _i32(seg).contiguous()
     out = torch.empty(B, C, int(num_key_blocks), dtype=torch.float32, device=q.device)
     a = _lib.BlockMaxArgs()
-    a.q = q.data_ptr(); a.q_sb, a.q_sc = q.stride(0), q.stride(1)
-    a.k = k.data_ptr(); a.k_sb, a.k_sk = k.stride(0), k.stride(1)
-    a.pos = posi.data_ptr(); a.pos_sb, a.pos_sc = posi.stride(0), posi.stride(1)
+    a.q = q.data_ptr(); a.q_sb, a.q_sc = q.stride()[:2]
+    a.k = k.data_ptr(); a.k_sb, a.k_sk = k.stride()[:2]
+    a.pos = posi.data_ptr(); a.pos_sb, a.pos_sc = posi.stride()[:2]
     if segi is not None:
-        a.seg = segi.data_ptr(); a.seg_sb, a.seg_sc = segi.stride(0), segi.stride(1)
-    a.out = out.data_ptr(); a.o_sb, a.o_sc, a.o_sn = out.stride(0), out.stride(1), out.stride(2)
+        a.seg = segi.data_ptr(); a.seg_sb, a.seg_sc = segi.stride()[:2]
+    a.out = out.data_ptr(); a.o_sb, a.o_sc, a.o_sn = out.stride()[:3]
     a.B, a.C, a.Sk, a.D, a.nblk = B, C, Sk, D, int(num_key_blocks)
     a.block_size, a.local_window = int(block_size), max(1, int(local_window))
     a.dtype = _lib.dtype_code(q.dtype)
