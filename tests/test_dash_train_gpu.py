@@ -204,3 +204,27 @@ def test_dash_train_patch_rebinds_and_host_fallback(dev):
         patch.restore(mod)
         del sys.modules[dash_mod.__name__]
     assert DashAttention()._route(None, None) == "eager-route"
+
+
+@pytest.mark.parametrize("nblk", [1, 2, 63, 64, 65, 256, 257, 1024, 1025, 3000])
+def test_entmax_threshold_row_shapes(dev, nblk):
+    """The prior of rows whose threshold sits at either end of its range, at
+    the register kernels' edges (256, 1024 blocks per row): every score equal,
+    nearly equal, one far above the rest, two equal leaders, an even ramp, and
+    normal ones of several spreads.  Bar 1e-6: tau is known to 1e-12, and the
+    fp32 z (below 1 where it counts) and its square round by 6e-8 each."""
+    from srswa import dash_train as DT
+    g = torch.Generator().manual_seed(nblk)
+    rows = [torch.zeros(nblk), torch.randn(nblk, generator=g) * 1e-4, torch.randn(nblk, generator=g) * 0.1,
+            torch.randn(nblk, generator=g), torch.randn(nblk, generator=g) * 20,
+            torch.linspace(-1, 1, nblk), torch.linspace(0, 1e-3, nblk)]
+    lead = torch.randn(nblk, generator=g) * 0.2
+    lead[0] = 9.0
+    pair = lead.clone()
+    pair[-1] = 9.0
+    sc = torch.stack(rows + [lead, pair])[None]
+    prior, cand = DT.route_forward(sc.to(dev), None, None, 1.0, -1.0e4)
+    ref, rc = O.dash_route_train(sc.double(), None, None, 1.0)
+    err = (prior.cpu().double() - ref).abs().max().item()
+    report(f"[err] entmax threshold, {nblk} blocks: max-abs {err:.2e} (bar 1e-6)")
+    assert torch.equal(cand.cpu(), rc) and err <= 1e-6

@@ -8,12 +8,11 @@
 // where the reference's tensors do (bf16 training runs the whole router in
 // bf16); reductions accumulate in fp32, the entmax threshold in fp64:
 //   route:  candidates (score > -5e8, under the row's block / image mask,
-//           falling back to every remote block), x, z = (x - max) / 2; the z
-//           above -1 (every support member: tau >= max z - 1) are compacted and
-//           sorted descending (bitonic: across the wave when at most 64, else
-//           in LDS), their fp64 prefix sums give each
-//           rank's closed-form threshold tau_r = mean - sqrt(max((1 - ss) / r,
-//           0)), support = #{r : tau_r <= z_(r)}, prior = max(z - tau_support, 0)^2;
+//           falling back to every remote block), x, z = (x - max) / 2; the
+//           entmax threshold tau, sum max(z - tau, 0)^2 = 1, by Newton's steps
+//           over the z above -1 (every support member: tau >= max z - 1) and
+//           the closed form mean - sqrt(max((1 - ss) / r, 0)) over the r of
+//           them above it; prior = max(z - tau, 0)^2;
 //   select: the top K of the 64-bit keys (order key of the masked prior,
 //           ~block id) by a lane-maximum threshold and a wave sort, then the
 //           bias of the K slots by wave reductions;
@@ -75,88 +74,53 @@ __device__ __forceinline__ float route_x(const srswa_dash_route_train_args& a, f
   return x;
 }
 
-// Sort the c (<= pcap) floats of s_z descending in LDS (bitonic over the
-// next power of two >= max(c, 64), padded with -inf); one wave per workgroup.
-__device__ __forceinline__ int lds_sort_desc(float* s_z, int c, int lane) {
-  int P = kWave;
-  while (P < c) P <<= 1;
-  for (int i = c + lane; i < P; i += kWave) s_z[i] = -INFINITY;
-  __syncthreads();
-  for (int k = 2; k <= P; k <<= 1) {
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      for (int t = lane; t < P / 2; t += kWave) {
-        const int i = 2 * j * (t / j) + (t % j), l = i + j;
-        const float vi = s_z[i], vl = s_z[l];
-        const bool desc = (i & k) == 0;
-        if (desc ? (vi < vl) : (vi > vl)) {
-          s_z[i] = vl;
-          s_z[l] = vi;
-        }
-      }
-      __syncthreads();
-    }
+// tau of the z above -1 (each_z(f) calls f on every one this lane holds),
+// without sorting them.  sqrt(sum max(z - t, 0)^2) - 1 is convex and falls in
+// t, so Newton's steps from t = -1, left of the root (the largest z is 0),
+// stay left of it and reach it in a few; the closed form over the z above the
+// last t then gives tau in fp64.  t ends within 1e-6 of the root: a z that
+// close to it on the wrong side changes the closed form by its square.
+template <typename Each>
+__device__ __forceinline__ double entmax_threshold(Each&& each_z) {
+  float t = -1.f;
+  for (int it = 0; it < 64; ++it) {
+    float f = 0.f, r = 0.f;
+    each_z([&](float z) __attribute__((always_inline)) {
+      const float p = fmaxf(z - t, 0.f);
+      f = fmaf(p, p, f);
+      r += p;
+    });
+    f = wave_sum(f);
+    if (!(f > 1.f + 1e-6f)) break;
+    const float nt = t + (f - sqrtf(f)) / wave_sum(r);
+    if (!(nt > t)) break;
+    t = nt;
   }
-  return P;
-}
-
-// tau of the c largest z, sorted descending: E per lane in s_z (lane-major),
-// or one per lane in `mine` (E == 0)
-__device__ __forceinline__ double entmax_threshold(const float* s_z, float mine, int c, int E, int lane) {
-  const int per = E > 0 ? E : 1;
-  auto val = [&](int e) __attribute__((always_inline)) { return E > 0 ? (double)s_z[lane * E + e] : (double)mine; };
-  double l1 = 0.0, l2 = 0.0;
-  for (int e = 0; e < per; ++e)
-    if (lane * per + e < c) {
-      const double v = val(e);
-      l1 += v;
-      l2 += v * v;
-    }
-  double i1 = l1, i2 = l2;                          // inclusive scan over lanes
-#pragma unroll
-  for (int o = 1; o < kWave; o <<= 1) {
-    const double t1 = __shfl_up(i1, o, kWave), t2 = __shfl_up(i2, o, kWave);
-    if (lane >= o) {
-      i1 += t1;
-      i2 += t2;
-    }
-  }
-  double b1 = __shfl_up(i1, 1, kWave), b2 = __shfl_up(i2, 1, kWave);
-  if (lane == 0) b1 = b2 = 0.0;
-  // support = #{ranks r with tau_r <= z_(r)}; tau_r of every rank this lane holds
-  int cnt = 0;
-  double s1 = b1, s2 = b2;
-  for (int e = 0; e < per; ++e)
-    if (lane * per + e < c) {
-      const double v = val(e);
-      s1 += v;
-      s2 += v * v;
-      cnt += entmax_tau(s1, s2, lane * per + e + 1) <= v ? 1 : 0;
-    }
-  const int support = max(wave_sum_int(cnt), 1);
-  const int owner = (support - 1) / per;
-  double tau = 0.0;
-  if (lane == owner) {
-    s1 = b1;
-    s2 = b2;
-    for (int e = 0; lane * per + e < support; ++e) {
-      const double v = val(e);
-      s1 += v;
-      s2 += v * v;
-    }
-    tau = entmax_tau(s1, s2, support);
-  }
-  return __shfl(tau, owner, kWave);
+  double s1 = 0.0, s2 = 0.0;
+  int c = 0;
+  each_z([&](float z) __attribute__((always_inline)) {
+    const bool in = z > t;
+    const double v = in ? (double)z : 0.0;
+    s1 += v;
+    s2 += v * v;
+    c += in ? 1 : 0;
+  });
+  return entmax_tau(wave_sum_f64(s1), wave_sum_f64(s2), max(wave_sum_int(c), 1));
 }
 
 // NPL > 0: the row's scores and mask bits stay in registers (block i = lane +
-// 64 t); NPL == 0 re-reads the row for every pass (rows above 1024 blocks).
-// The z above -1 (usually few) are sorted across the wave when at most 64,
-// else in LDS.
+// 64 t), four rows per workgroup; NPL == 0 (rows above 1024 blocks) re-reads
+// the row for every pass, one row per workgroup, and keeps the z above -1
+// (usually few) in LDS.
+// Each row is a chain of reductions, not a stream: 32,768 rows of 256 fp32
+// scores, 75 MB, took 87 us with every z above -1 (flat scores) and 37 us with
+// few, the z sorted and prefix-summed; Newton's steps take 34 and 29 us.
 template <typename T, int NPL>
-__global__ __launch_bounds__(kWave) void route_train_kernel(srswa_dash_route_train_args a, int pcap) {
-  extern __shared__ float s_z[];                    // [pcap]
-  const int lane = threadIdx.x;
-  const int64_t row = blockIdx.x;
+__global__ __launch_bounds__(NPL > 0 ? 4 * kWave : kWave) void route_train_kernel(srswa_dash_route_train_args a) {
+  extern __shared__ float s_z[];                    // NPL == 0: [nblk]
+  const int lane = threadIdx.x % kWave;
+  const int64_t row = NPL > 0 ? (int64_t)blockIdx.x * 4 + threadIdx.x / kWave : (int64_t)blockIdx.x;
+  if (row >= a.rows) return;
   const int n = a.nblk;
   const void* sr = reinterpret_cast<const char*>(a.scores) + row * a.sc_sr * (int64_t)sizeof(T);
   const uint8_t* bc = a.block_cand ? a.block_cand + row * a.bc_sr : nullptr;
@@ -209,49 +173,35 @@ __global__ __launch_bounds__(kWave) void route_train_kernel(srswa_dash_route_tra
   }
   xm = wave_max(xm);
 
-  // z = (x - max) / 2 (kept in sv for NPL > 0), cand written, the z > -1 counted
+  // z = (x - max) / 2 (kept in sv for NPL > 0, those above -1 in LDS otherwise), cand written
   uint8_t* cr = a.cand + row * a.c_sr;
-  int cnt_hi = 0;
+  int c = 0;                                        // NPL == 0: z in LDS
   for (int t = 0; t < nt; ++t) {
     const int i = lane + kWave * t;
+    float z = -INFINITY;
     if (i < n) {
       bool cd;
-      const float z = rnd<T>(route_x<T>(a, score(t, i), !use_mask || maskb(t, i), cd) - xm) * 0.5f;
+      z = rnd<T>(route_x<T>(a, score(t, i), !use_mask || maskb(t, i), cd) - xm) * 0.5f;
       cr[i] = cd ? 1 : 0;
-      cnt_hi += z > -1.f ? 1 : 0;
-      if constexpr (NPL > 0) sv[t] = z;
     }
-  }
-  const int c = wave_sum_int(cnt_hi);
-  // compaction of the z > -1 into s_z (ascending block order)
-  {
-    int base = 0;
-    for (int t = 0; t < nt; ++t) {
-      const int i = lane + kWave * t;
-      float z = -INFINITY;
-      if (i < n) {
-        if constexpr (NPL > 0) {
-          z = sv[t];
-        } else {
-          bool cd;
-          z = rnd<T>(route_x<T>(a, score(t, i), !use_mask || maskb(t, i), cd) - xm) * 0.5f;
-        }
-      }
+    if constexpr (NPL > 0) {
+      sv[t] = z;                                    // -inf past the row: in no sum
+    } else {
       const bool keep = z > -1.f;
       const uint64_t bal = __ballot(keep);
-      if (keep) s_z[base + __popcll(bal & ((1ull << lane) - 1ull))] = z;
-      base += __popcll(bal);
+      if (keep) s_z[c + __popcll(bal & ((1ull << lane) - 1ull))] = z;
+      c += __popcll(bal);
     }
   }
-  double tau;
-  if (c <= kWave) {
-    __syncthreads();
-    const float mine = wave_sort_desc<float>(lane < c ? s_z[lane] : -INFINITY, lane);
-    tau = entmax_threshold(nullptr, mine, c, 0, lane);
-  } else {
-    const int P = lds_sort_desc(s_z, c, lane);
-    tau = entmax_threshold(s_z, 0.f, c, P / kWave, lane);
-  }
+  if constexpr (NPL == 0) __syncthreads();
+  const double tau = entmax_threshold([&](auto&& f) __attribute__((always_inline)) {
+    if constexpr (NPL > 0) {
+#pragma unroll
+      for (int t = 0; t < NPL; ++t) f(sv[t]);
+    } else {
+      for (int i = lane; i < c; i += kWave) f(s_z[i]);
+    }
+  });
 
   void* pr = reinterpret_cast<char*>(a.prior) + row * a.p_sr * (int64_t)sizeof(T);
   for (int t = 0; t < nt; ++t) {
@@ -468,14 +418,14 @@ int check_dtype(int dtype, const char* what) {
 constexpr int kMaxBlocks = 8192;    // LDS row of one wavefront: 32 KB
 
 template <typename T>
-void launch_route(const srswa_dash_route_train_args& a, int pcap, hipStream_t s) {
-  const size_t lds = (size_t)pcap * sizeof(float);
+void launch_route(const srswa_dash_route_train_args& a, hipStream_t s) {
+  const dim3 quads((unsigned)ceil_div(a.rows, 4));
   if (a.nblk <= 4 * kWave)
-    hipLaunchKernelGGL((route_train_kernel<T, 4>), dim3(a.rows), dim3(kWave), lds, s, a, pcap);
+    hipLaunchKernelGGL((route_train_kernel<T, 4>), quads, dim3(4 * kWave), 0, s, a);
   else if (a.nblk <= 16 * kWave)
-    hipLaunchKernelGGL((route_train_kernel<T, 16>), dim3(a.rows), dim3(kWave), lds, s, a, pcap);
+    hipLaunchKernelGGL((route_train_kernel<T, 16>), quads, dim3(4 * kWave), 0, s, a);
   else
-    hipLaunchKernelGGL((route_train_kernel<T, 0>), dim3(a.rows), dim3(kWave), lds, s, a, pcap);
+    hipLaunchKernelGGL((route_train_kernel<T, 0>), dim3(a.rows), dim3(kWave), (size_t)a.nblk * sizeof(float), s, a);
 }
 
 int launch_status(const char* what) {
@@ -508,12 +458,10 @@ extern "C" int srswa_dash_route_train(const srswa_dash_route_train_args* a, void
     return SRSWA_UNSUPPORTED;
   }
   if (a->rows == 0 || a->nblk == 0) return SRSWA_OK;
-  int pcap = kWave;
-  while (pcap < a->nblk) pcap <<= 1;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (a->dtype == SRSWA_F32) launch_route<float>(*a, pcap, s);
-  else if (a->dtype == SRSWA_BF16) launch_route<bf16_t>(*a, pcap, s);
-  else launch_route<__half>(*a, pcap, s);
+  if (a->dtype == SRSWA_F32) launch_route<float>(*a, s);
+  else if (a->dtype == SRSWA_BF16) launch_route<bf16_t>(*a, s);
+  else launch_route<__half>(*a, s);
   return launch_status("dash route train");
 }
 
