@@ -74,57 +74,6 @@ __device__ __forceinline__ F32x8 f32x8(const float* v) {
                make_uint4(__float_as_uint(v[4]), __float_as_uint(v[5]), __float_as_uint(v[6]), __float_as_uint(v[7]))};
 }
 
-// fp32 products on the 16-bit matrix cores.  A finite fp32 value is the exact
-// sum of three bf16 values, each the rounding of what the ones before it leave
-// (8 + 8 + 8 significant bits), so a product of two values is nine bf16
-// products, exact in fp32.  The six largest are taken; the three left out are
-// below 2^-26 of |a||b| together, a quarter of an fp32 rounding of the product
-// itself.  Six v_mfma_f32_32x32x16_bf16 replace eight v_mfma_f32_32x32x2_f32
-// of eight times their length per flop: 192 cycles instead of 512.
-struct Split3 {
-  uint4 p[3];   // 8 values each: leading, middle and last part
-};
-__device__ __forceinline__ void split_pair(float a, float b, uint32_t& w0, uint32_t& w1, uint32_t& w2) {
-  // the empty asm keeps the compiler from converting each value a second time
-  // for the residual instead of taking it from the packed word
-  w0 = pack_bf16x2(a, b);
-  asm("" : "+v"(w0));
-  const float ra = a - bf16_lo(w0), rb = b - bf16_hi(w0);
-  w1 = pack_bf16x2(ra, rb);
-  asm("" : "+v"(w1));
-  w2 = pack_bf16x2(ra - bf16_lo(w1), rb - bf16_hi(w1));
-}
-__device__ __forceinline__ Split3 split8(const float4& x, const float4& y) {
-  Split3 s;
-  split_pair(x.x, x.y, s.p[0].x, s.p[1].x, s.p[2].x);
-  split_pair(x.z, x.w, s.p[0].y, s.p[1].y, s.p[2].y);
-  split_pair(y.x, y.y, s.p[0].z, s.p[1].z, s.p[2].z);
-  split_pair(y.z, y.w, s.p[0].w, s.p[1].w, s.p[2].w);
-  return s;
-}
-// The parts hold a value exactly only while they stay normal and the leading
-// one does not round to infinity, and a sum of products must not overflow on
-// the way: |x| at most 2^59 (128 products stay below 2^125), and values whose
-// last part is lost below 2^-126 only beside larger ones.  A caller gathers
-// the largest magnitude of a group of values and takes the fp32 form for a
-// group outside these bounds (NaN spreads through the parts by itself).
-__device__ __forceinline__ float max_abs4(float m, const float4& v) {
-  return fmaxf(fmaxf(fmaxf(m, fabsf(v.x)), fmaxf(fabsf(v.y), fabsf(v.z))), fabsf(v.w));
-}
-__device__ __forceinline__ bool split_safe(float maxabs) {
-  return maxabs == 0.f || (maxabs >= 0x1p-90f && maxabs <= 0x1p+59f);
-}
-// c += the leading product, e += the five smaller ones: their roundings stay
-// 2^-8 of the sum's, and the sum itself is rounded once per 16-wide step
-__device__ __forceinline__ void mac_split(const Split3& a, const Split3& b, f32x16_t& c, f32x16_t& e) {
-  c = Mfma<bf16_t>::mac(a.p[0], b.p[0], c);
-  e = Mfma<bf16_t>::mac(a.p[2], b.p[0], e);
-  e = Mfma<bf16_t>::mac(a.p[0], b.p[2], e);
-  e = Mfma<bf16_t>::mac(a.p[1], b.p[1], e);
-  e = Mfma<bf16_t>::mac(a.p[1], b.p[0], e);
-  e = Mfma<bf16_t>::mac(a.p[0], b.p[1], e);
-}
-
 // The fp32 A operand X^T (M = feature d, K = 16 rows of X) in the key order of
 // the MFMA output rows that form the B operand: lane (d = l % 32, h) value j
 // is X[r0 + 4h + j][c0 + d] for j < 4 and X[r0 + 8 + 4h + (j - 4)][c0 + d]

@@ -48,14 +48,13 @@
 // workgroup), hc_summary_bwd (one workgroup per block: the partials summed in
 // a fixed chunk order, stage 0 redone, then its backward), and hc_dhc_reduce
 // (block partials of d head_cls summed in a fixed order);
-// bm_fwd (128 rows per workgroup, 64-key chunks through LDS, S^T = K Q^T as six
-// bf16 products of three-part fp32 operands, then per block the
+// bm_fwd (128 rows per workgroup, 64-key chunks through LDS, S^T = K Q^T on
+// v_mfma_f32_32x32x2_f32 as the inference block-max kernel, then per block the
 // clamped max, its tie and in-range masks), bm_bwd_dq (4 rows per wave, 16
 // waves per 64-row tile, the arg-max key rows of two blocks gathered
 // together) and bm_bwd_dk (four keys per wave, 16 lanes each, scanning the
 // block's codes in row order).  No atomics: every result is deterministic.
 #include <algorithm>
-#include <climits>
 #include <type_traits>
 
 #include "mfma_common.h"
@@ -673,7 +672,7 @@ __global__ __launch_bounds__(kDhcDims * kDhcParts) void hc_dhc_reduce_kernel(HcB
 // ---------------------------------------------------------------- block max
 constexpr int kBmRows = 128;                 // query rows per workgroup (4 waves of 32)
 constexpr int kBmThreads = 2 * kBmRows;
-constexpr int kBmSlab = 16;                 // chunks of 64 keys per workgroup
+constexpr int kBmSlab = 16;                  // chunks of 64 keys per workgroup
 constexpr int kCodeMulti = 1 << 16;          // several keys take the gradient: mask in the side array
 constexpr int kCodeNone = 1 << 17;           // no key takes the gradient
 
@@ -682,72 +681,40 @@ struct BmK {
   int ntiles, nslab;
 };
 
-// S^T tile (32 keys x 32 rows) straight from memory on the fp32 matrix cores,
-// for operands that split_safe() refuses: lane half h supplies head dims
-// 8 m + 4 h .. + 3 of step group m to both operands
+// S^T tile (32 keys x 32 rows) from the staged chunk, fp32 operands: lane half
+// h supplies head dims 8 m + 4 h .. + 3 of step group m to both operands
 template <int D>
-__device__ __forceinline__ f32x16_t bm_tile_f32(const float* krow, const float* qrow, int h) {
+__device__ __forceinline__ f32x16_t bm_tile(const float* sK, int key, const float4* qf, int h) {
+  constexpr int KP = D + 4;
   f32x16_t s = zero16();
-#pragma unroll 2
+#pragma unroll
   for (int m = 0; m < D / 8; ++m) {
-    const float4 kv = *reinterpret_cast<const float4*>(krow + 8 * m + 4 * h);
-    const float4 qv = *reinterpret_cast<const float4*>(qrow + 8 * m + 4 * h);
-    s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.x, qv.x, s, 0, 0, 0);
-    s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.y, qv.y, s, 0, 0, 0);
-    s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.z, qv.z, s, 0, 0, 0);
-    s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.w, qv.w, s, 0, 0, 0);
+    const float4 kv = *reinterpret_cast<const float4*>(sK + key * KP + 8 * m + 4 * h);
+    s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.x, qf[m].x, s, 0, 0, 0);
+    s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.y, qf[m].y, s, 0, 0, 0);
+    s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.z, qf[m].z, s, 0, 0, 0);
+    s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.w, qf[m].w, s, 0, 0, 0);
   }
   return s;
 }
 
-// the key bits (32 half + 8 (r / 4) + 4 h + r % 4) of a lane's own bits
-// 16 half + r of its S^T tiles
-__device__ __forceinline__ uint32_t spread_nibbles(uint32_t v) {
-  v = (v | (v << 8)) & 0x00ff00ffu;
-  return (v | (v << 4)) & 0x0f0f0f0fu;
-}
-__device__ __forceinline__ uint64_t key_bits(uint32_t own, int h) {
-  const uint64_t v = (uint64_t)spread_nibbles(own & 0xffffu) | ((uint64_t)spread_nibbles(own >> 16) << 32);
-  return h ? v << 4 : v;
-}
-__device__ __forceinline__ uint64_t xor32_or(uint64_t v) {
-  const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)v, (uint32_t)v, false, false);
-  const auto hi = __builtin_amdgcn_permlane32_swap((uint32_t)(v >> 32), (uint32_t)(v >> 32), false, false);
-  return ((uint64_t)(hi[0] | hi[1]) << 32) | (lo[0] | lo[1]);
+__device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int m) {
+  const uint32_t lo = __shfl_xor((uint32_t)v, m, kWave), hi = __shfl_xor((uint32_t)(v >> 32), m, kWave);
+  return ((uint64_t)hi << 32) | lo;
 }
 
-// Bound by the matrix cores and the VALU work beside them.  S^T = K Q^T of fp32
-// operands as six products of their bf16 parts (mfma_common.h, Split3): the
-// row's parts live in registers (96 for D = 128), a chunk's are made from the
-// fp32 keys as they are staged, and the fragments of the next six MFMAs are
-// read under the present six.  Two workgroups share a CU (61 KB of LDS, 256
-// registers each), so that one converts and takes block maxima while the other
-// multiplies.  Measured at B = 2, S = 16384, D = 128, 64-key blocks (64.5
-// GFLOP): 434 us, 149 TFLOP/s of fp32 products, against 1246 us on
-// v_mfma_f32_32x32x2_f32 (52 TFLOP/s); of that, 177 us came with dealing row
-// tiles instead of slabs to the XCDs.  Slabs of 8 and 5 chunks: 451 and 487.
 template <int D, int BS>
 __global__ __launch_bounds__(kBmThreads, 2) void bm_fwd_kernel(BmK p) {
-  constexpr int KP = D + 8;                       // bf16 elements per staged key row and part
+  constexpr int KP = D + 4;
   constexpr int NSUB = kChunk / BS;
-  constexpr int NQ = D / 16;
-  constexpr bool kStageZ = NSUB <= 2;             // scores staged in LDS, written once per slab
-  constexpr int ZP = kBmSlab * NSUB + 1;
-  __shared__ __align__(16) uint16_t sK[3 * kChunk * KP];
-  __shared__ float s_z[kStageZ ? kBmRows * ZP : 1];
-  __shared__ int s_maxls, s_bad[2];
+  __shared__ __align__(16) float sK[kChunk * KP];
+  __shared__ int s_maxls;
   const srswa_bm_score_args& a = p.a;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
   const int h = lane / 32, rl = lane % 32;
-  // workgroups are dealt to the eight XCDs round-robin: an XCD takes every
-  // eighth row tile with all its slabs (a causal row tile reaches only the
-  // slabs before it, so dealing by slab left the XCDs of the last slabs idle),
-  // the tile fastest, so that its L2 serves a slab's keys to all of them
-  const int tpx = ceil_div(a.B * p.ntiles, 8);
-  const int bt = ((int)(blockIdx.x >> 3) % tpx) * 8 + (int)(blockIdx.x & 7);
-  const int slab = (int)(blockIdx.x >> 3) / tpx;
-  if (bt >= a.B * p.ntiles) return;
-  const int tile = bt % p.ntiles;
+  const int slab = blockIdx.x % p.nslab;
+  const int bt = blockIdx.x / p.nslab;
+  const int tile = p.ntiles - 1 - bt % p.ntiles;   // heaviest (last rows) first
   const int b = bt / p.ntiles;
   const int row = tile * kBmRows + wave * 32 + rl;
   const bool row_ok = row < a.S;
@@ -756,11 +723,9 @@ __global__ __launch_bounds__(kBmThreads, 2) void bm_fwd_kernel(BmK p) {
     const int pos = a.pos[(int64_t)b * a.pos_sb + (int64_t)row * a.pos_st];
     ls = min(max(pos - a.local_window + 1, 0), a.S);
   }
-  const int wlo = wave_min_int(row_ok ? ls : INT_MAX);   // chunks below are scored whole by every row of the wave
-  const int whi = wave_max_int(ls);                      // chunks at or past hold no remote key of the wave
-  if (tid == 0) s_maxls = s_bad[0] = s_bad[1] = 0;
+  if (tid == 0) s_maxls = 0;
   __syncthreads();
-  if (lane == 0) atomicMax(&s_maxls, whi);
+  if (row_ok && h == 0) atomicMax(&s_maxls, ls);
   __syncthreads();
   const int nchunks = ceil_div(s_maxls, kChunk);
   const int c_lo = slab * kBmSlab;
@@ -768,181 +733,88 @@ __global__ __launch_bounds__(kBmThreads, 2) void bm_fwd_kernel(BmK p) {
   const int blk_lo = c_lo * NSUB;
   const int blk_hi = slab == p.nslab - 1 ? a.nblk : min(a.nblk, (c_lo + kBmSlab) * NSUB);
 
+  float4 qf[D / 8];
+  {
+    const float* qrow = a.q + (int64_t)b * a.q_sb + (int64_t)(row_ok ? row : 0) * a.q_st;
+#pragma unroll
+    for (int m = 0; m < D / 8; ++m)
+      qf[m] = row_ok ? *reinterpret_cast<const float4*>(qrow + 8 * m + 4 * h) : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
   float* zrow = a.z + (int64_t)b * a.z_sb + (int64_t)(row_ok ? row : 0) * a.z_st;
   int32_t* code = a.code + (int64_t)b * a.nblk * a.S + (row_ok ? row : 0);      // [b][blk][row]
   uint64_t* tm = a.tiemask + ((int64_t)b * a.S + (row_ok ? row : 0)) * a.nblk;   // [b][row][blk]
   const float* kg = a.k + (int64_t)b * a.k_sb;
-  const float* qrow = a.q + (int64_t)b * a.q_sb + (int64_t)(row_ok ? row : 0) * a.q_st;
-  if (c_lo < c_hi) {
-    constexpr int PR = D / 8;                       // 8-value pieces per key row
-    constexpr int PPT = kChunk * PR / kBmThreads;   // per thread
-    float4 pre[PPT][2];
-    // piece i of a thread: key row tid / PR + i kBmThreads / PR, so the lane's part of every address is one offset
-    const int64_t lane_off = (int64_t)(tid / PR) * a.k_st + 8 * (tid % PR);
-    auto fetch = [&](int c) {
-      const bool full = (c + 1) * kChunk <= a.S;
+  constexpr int PR = D / 4;                       // 16-byte pieces per key row
+  constexpr int PPT = kChunk * PR / kBmThreads;   // per thread
+  float4 pre[PPT];
+  auto fetch = [&](int c) {
 #pragma unroll
-      for (int i = 0; i < PPT; ++i) {
-        const int r0 = c * kChunk + i * (kBmThreads / PR);
-        const float* src = kg + (int64_t)r0 * a.k_st + lane_off;
-        if (!full)                                    // keys past the last repeat it: they are never live
-          src = kg + (int64_t)min(r0 + tid / PR, a.S - 1) * a.k_st + 8 * (tid % PR);
-        pre[i][0] = *reinterpret_cast<const float4*>(src);
-        pre[i][1] = *reinterpret_cast<const float4*>(src + 4);
-      }
-    };
-    fetch(c_lo);
-    Split3 qf[NQ];
-    bool qsafe;
-    {
-      float m = 0.f;
-#pragma unroll
-      for (int ks = 0; ks < NQ; ++ks) {
-        const float4 x = *reinterpret_cast<const float4*>(qrow + 16 * ks + 8 * h);
-        const float4 y = *reinterpret_cast<const float4*>(qrow + 16 * ks + 8 * h + 4);
-        m = max_abs4(max_abs4(m, x), y);
-        qf[ks] = split8(x, y);
-      }
-      qsafe = __all(split_safe(m));
+    for (int i = 0; i < PPT; ++i) {
+      const int pc = tid + kBmThreads * i;
+      const int j = c * kChunk + pc / PR, col = pc % PR;
+      pre[i] = j < a.S ? *reinterpret_cast<const float4*>(kg + (int64_t)j * a.k_st + 4 * col)
+                       : make_float4(0.f, 0.f, 0.f, 0.f);
     }
-    for (int c = c_lo; c < c_hi; ++c) {
-      const int j0 = c * kChunk;
-      Split3 pl[PPT];
-      float m = 0.f;
+  };
+  if (c_lo < c_hi) fetch(c_lo);
+  for (int c = c_lo; c < c_hi; ++c) {
+    const int j0 = c * kChunk;
+    __syncthreads();
 #pragma unroll
-      for (int i = 0; i < PPT; ++i) {
-        m = max_abs4(max_abs4(m, pre[i][0]), pre[i][1]);
-        pl[i] = split8(pre[i][0], pre[i][1]);
-      }
-      if (c + 1 < c_hi) fetch(c + 1);
-      lds_barrier();                                // the previous chunk is consumed
+    for (int i = 0; i < PPT; ++i) {
+      const int pc = tid + kBmThreads * i;
+      *reinterpret_cast<float4*>(sK + (pc / PR) * KP + (pc % PR) * 4) = pre[i];
+    }
+    __syncthreads();
+    if (c + 1 < c_hi) fetch(c + 1);
+    const f32x16_t s0 = bm_tile<D>(sK, rl, qf, h);
+    const f32x16_t s1 = bm_tile<D>(sK, 32 + rl, qf, h);
 #pragma unroll
-      for (int i = 0; i < PPT; ++i) {
-        const int pc = tid + kBmThreads * i;
-        uint16_t* dst = sK + (pc / PR) * KP + 8 * (pc % PR);
+    for (int sb = 0; sb < NSUB; ++sb) {
+      float mx = -INFINITY;
 #pragma unroll
-        for (int t = 0; t < 3; ++t) *reinterpret_cast<uint4*>(dst + t * kChunk * KP) = pl[i].p[t];
-      }
-      if (!__all(split_safe(m)) && lane == 0) s_bad[c & 1] = 1;
-      lds_barrier();
-      const bool safe = qsafe && s_bad[c & 1] == 0;
-      if (tid == 0) s_bad[(c + 1) & 1] = 0;         // set again only past the next barrier
-      f32x16_t s0, s1;
-      if (safe) {
-        f32x16_t e0 = zero16(), e1 = zero16();
-        s0 = s1 = zero16();
-        // six MFMAs per (step, key half); the next one's three fragments are read under them
-        auto frag = [&](int n) __attribute__((always_inline)) {   // n = 2 step + half
-          Split3 f;
-          const uint16_t* src = sK + (rl + 32 * (n & 1)) * KP + 16 * (n >> 1) + 8 * h;
+      for (int r = 0; r < 16; ++r)
 #pragma unroll
-          for (int t = 0; t < 3; ++t) f.p[t] = *reinterpret_cast<const uint4*>(src + t * kChunk * KP);
-          return f;
-        };
-        Split3 k0 = frag(0);
-#pragma unroll
-        for (int n = 0; n < 2 * NQ; ++n) {
-          Split3 kn = k0;
-          if (n + 1 < 2 * NQ) kn = frag(n + 1);
-          if (n & 1) mac_split(k0, qf[n >> 1], s1, e1);
-          else mac_split(k0, qf[n >> 1], s0, e0);
-          k0 = kn;
+        for (int half = 0; half < 2; ++half) {
+          const int off = 32 * half + d_row(r, h);
+          if (off / BS == sb && j0 + off < ls) mx = fmaxf(mx, clamp_act(half ? s1[r] : s0[r]));
         }
-        __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+      mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+      uint64_t tie = 0, grad = 0;                 // block-relative key bits
 #pragma unroll
-        for (int n = 0; n < 2 * NQ; ++n) {
-          if (n + 1 < 2 * NQ) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);   // reads of the next
-          __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);                       // MFMAs of this one
-        }
+      for (int r = 0; r < 16; ++r)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          s0[r] += e0[r];
-          s1[r] += e1[r];
-        }
-      } else {
-        s0 = bm_tile_f32<D>(kg + (int64_t)min(j0 + rl, a.S - 1) * a.k_st, qrow, h);
-        s1 = bm_tile_f32<D>(kg + (int64_t)min(j0 + 32 + rl, a.S - 1) * a.k_st, qrow, h);
-      }
-      // a lane's scores 16 half + r in one array; block sb of the chunk holds those with sub(i) == sb
-      auto val = [&](int i) __attribute__((always_inline)) { return i < 16 ? s0[i] : s1[i - 16]; };
-      auto sub = [](int i) __attribute__((always_inline)) {
-        return NSUB == 1 ? 0 : NSUB == 2 ? i / 16 : i / 8;
-      };
-      float mx[NSUB];
-      uint32_t tie = 0, grad = 0;                   // own bits
-      bool inside = j0 + kChunk <= wlo;
-      if (inside) {
-        // every key live: the largest score, clamped (the clamp is monotone)
-#pragma unroll
-        for (int sb = 0; sb < NSUB; ++sb) mx[sb] = -kActClamp;
-#pragma unroll
-        for (int i = 0; i < 32; ++i) mx[sub(i)] = fmaxf(mx[sub(i)], val(i));
-        bool in = true;
-#pragma unroll
-        for (int sb = 0; sb < NSUB; ++sb) {
-          mx[sb] = xor32_max(mx[sb]);
-          in = in && fabsf(mx[sb]) < kActClamp;
-        }
-        inside = __all(in);
-        if (inside) {
-#pragma unroll
-          for (int i = 0; i < 32; ++i) tie |= val(i) == mx[sub(i)] ? 1u << i : 0u;
-          grad = tie;
-        }
-      }
-      if (!inside) {
-        const int lim = ls - j0 - 4 * h;            // score i is live when its key offset (less 4 h) is below
-        auto off = [](int i) __attribute__((always_inline)) { return 32 * (i / 16) + 8 * ((i % 16) >> 2) + (i & 3); };
-#pragma unroll
-        for (int sb = 0; sb < NSUB; ++sb) mx[sb] = -INFINITY;
-#pragma unroll
-        for (int i = 0; i < 32; ++i)
-          if (off(i) < lim) mx[sub(i)] = fmaxf(mx[sub(i)], clamp_act(val(i)));
-#pragma unroll
-        for (int sb = 0; sb < NSUB; ++sb) mx[sb] = xor32_max(mx[sb]);
-#pragma unroll
-        for (int i = 0; i < 32; ++i)
-          if (off(i) < lim && clamp_act(val(i)) == mx[sub(i)]) {
-            tie |= 1u << i;
-            if (clamp_act(val(i)) == val(i)) grad |= 1u << i;
-          }
-      }
-      const uint64_t tie64 = xor32_or(key_bits(tie, h)), grad64 = xor32_or(key_bits(grad, h));
-      if (row_ok && h == 0) {
-#pragma unroll
-        for (int sb = 0; sb < NSUB; ++sb) {
-          const int blk = c * NSUB + sb;
-          const uint64_t bm = BS == 64 ? ~0ull : (1ull << (BS % 64)) - 1ull;
-          const uint64_t tb = (tie64 >> (sb * BS % 64)) & bm, gb = (grad64 >> (sb * BS % 64)) & bm;
-          if (blk < a.nblk) {
-            const int ng = __popcll(gb);
-            int cd = kCodeNone;
-            if (ng > 0) cd = (int)__builtin_ctzll(gb) | (__popcll(tb) << 8) | (ng > 1 ? kCodeMulti : 0);
-            const float zv = mx[sb] == -INFINITY ? kScoreNeg : mx[sb];
-            if constexpr (kStageZ) s_z[(wave * 32 + rl) * ZP + blk - blk_lo] = zv;
-            else zrow[blk] = zv;
-            code[(int64_t)blk * a.S] = cd;
-            if (ng > 1) tm[blk] = gb;
+        for (int half = 0; half < 2; ++half) {
+          const int off = 32 * half + d_row(r, h);
+          if (off / BS == sb && j0 + off < ls) {
+            const float raw = half ? s1[r] : s0[r];
+            const float cv = clamp_act(raw);
+            const uint64_t bit = 1ull << (off - sb * BS);
+            if (cv == mx) {
+              tie |= bit;
+              if (raw == cv) grad |= bit;
+            }
           }
         }
+      tie |= shfl_xor_u64(tie, 32);
+      grad |= shfl_xor_u64(grad, 32);
+      const int blk = c * NSUB + sb;
+      if (row_ok && h == 0 && blk < a.nblk) {
+        const int ng = __popcll(grad);
+        int cd = kCodeNone;
+        if (ng > 0) cd = (int)__builtin_ctzll(grad) | (__popcll(tie) << 8) | (ng > 1 ? kCodeMulti : 0);
+        zrow[blk] = mx == -INFINITY ? kScoreNeg : mx;
+        code[(int64_t)blk * a.S] = cd;
+        if (ng > 1) tm[blk] = grad;
       }
     }
   }
-  const int done = max(c_hi > c_lo ? c_hi * NSUB : blk_lo, blk_lo);   // blocks at or past hold no remote key
-  if (row_ok && h == 0)
-    for (int blk = done; blk < blk_hi; ++blk) code[(int64_t)blk * a.S] = kCodeNone;
-  if constexpr (kStageZ) {
-    __syncthreads();
-    // 16 lanes per row: the slab's scores in runs of 64 bytes
-    for (int r = tid / 16; r < kBmRows; r += kBmThreads / 16) {
-      const int rw = tile * kBmRows + r;
-      if (rw >= a.S) break;
-      float* dst = a.z + (int64_t)b * a.z_sb + (int64_t)rw * a.z_st;
-      for (int blk = blk_lo + tid % 16; blk < blk_hi; blk += 16)
-        dst[blk] = blk < done ? s_z[r * ZP + blk - blk_lo] : kScoreNeg;
+  // the slab's blocks after the last visited chunk hold no remote key of any row
+  if (row_ok && h == 0) {
+    for (int blk = max(c_hi > c_lo ? c_hi * NSUB : blk_lo, blk_lo); blk < blk_hi; ++blk) {
+      zrow[blk] = kScoreNeg;
+      code[(int64_t)blk * a.S] = kCodeNone;
     }
-  } else if (row_ok && h == 0) {
-    for (int blk = done; blk < blk_hi; ++blk) zrow[blk] = kScoreNeg;
   }
 }
 
@@ -1363,7 +1235,7 @@ int bm_check(const srswa_bm_score_args* a, const char* what) {
 
 template <int D, int BS>
 void bm_launch_fwd(const BmK& k, hipStream_t st) {
-  const dim3 grid((unsigned)(((int64_t)k.a.B * k.ntiles + 7) / 8 * 8 * k.nslab));
+  const dim3 grid((unsigned)((int64_t)k.a.B * k.ntiles * k.nslab));
   hipLaunchKernelGGL((bm_fwd_kernel<D, BS>), grid, dim3(kBmThreads), 0, st, k);
 }
 
@@ -1411,7 +1283,7 @@ extern "C" int srswa_bm_score_fwd(const srswa_bm_score_args* a, void* stream) {
   k.a = *a;
   k.ntiles = ceil_div(a->S, kBmRows);
   k.nslab = std::max(1, ceil_div(ceil_div(a->S, kChunk), kBmSlab));
-  if (((int64_t)a->B * k.ntiles + 7) / 8 * 8 * k.nslab > 0x7fffffff) {
+  if ((int64_t)a->B * k.ntiles * k.nslab > 0x7fffffff) {
     set_error("block-max scores: grid too large");
     return SRSWA_UNSUPPORTED;
   }
