@@ -55,6 +55,7 @@
 // together) and bm_bwd_dk (four keys per wave, 16 lanes each, scanning the
 // block's codes in row order).  No atomics: every result is deterministic.
 #include <algorithm>
+#include <climits>
 #include <type_traits>
 
 #include "mfma_common.h"
@@ -672,7 +673,7 @@ __global__ __launch_bounds__(kDhcDims * kDhcParts) void hc_dhc_reduce_kernel(HcB
 // ---------------------------------------------------------------- block max
 constexpr int kBmRows = 128;                 // query rows per workgroup (4 waves of 32)
 constexpr int kBmThreads = 2 * kBmRows;
-constexpr int kBmSlab = 16;                  // chunks of 64 keys per workgroup
+constexpr int kBmSlab = 16;                 // chunks of 64 keys per workgroup
 constexpr int kCodeMulti = 1 << 16;          // several keys take the gradient: mask in the side array
 constexpr int kCodeNone = 1 << 17;           // no key takes the gradient
 
@@ -698,23 +699,51 @@ __device__ __forceinline__ f32x16_t bm_tile(const float* sK, int key, const floa
   return s;
 }
 
-__device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int m) {
-  const uint32_t lo = __shfl_xor((uint32_t)v, m, kWave), hi = __shfl_xor((uint32_t)(v >> 32), m, kWave);
-  return ((uint64_t)hi << 32) | lo;
+// the key bits (32 half + 8 (r / 4) + 4 h + r % 4) of a lane's own bits
+// 16 half + r of its S^T tiles
+__device__ __forceinline__ uint32_t spread_nibbles(uint32_t v) {
+  v = (v | (v << 8)) & 0x00ff00ffu;
+  return (v | (v << 4)) & 0x0f0f0f0fu;
+}
+__device__ __forceinline__ uint64_t key_bits(uint32_t own, int h) {
+  const uint64_t v = (uint64_t)spread_nibbles(own & 0xffffu) | ((uint64_t)spread_nibbles(own >> 16) << 32);
+  return h ? v << 4 : v;
+}
+__device__ __forceinline__ uint64_t xor32_or(uint64_t v) {
+  const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)v, (uint32_t)v, false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((uint32_t)(v >> 32), (uint32_t)(v >> 32), false, false);
+  return ((uint64_t)(hi[0] | hi[1]) << 32) | (lo[0] | lo[1]);
 }
 
+// Bound by the fp32 matrix cores.  Two workgroups of four waves share a CU, so
+// that one takes block maxima and stages keys while the other multiplies.  A
+// chunk whose keys are all live for every row of the wave takes its maxima from
+// the raw scores (the clamp is monotone) and its ties from one comparison per
+// score, and the scores leave through LDS in runs of a slab.  Measured at B = 2,
+// S = 16384, D = 128, 64-key blocks (64.5 GFLOP): 1246 -> 703 us, 92 TFLOP/s,
+// most of it from dealing row tiles instead of slabs to the XCDs.  Slabs of 8,
+// 12 and 24 chunks: 715, 698 and 728 us.
 template <int D, int BS>
 __global__ __launch_bounds__(kBmThreads, 2) void bm_fwd_kernel(BmK p) {
   constexpr int KP = D + 4;
   constexpr int NSUB = kChunk / BS;
+  constexpr bool kStageZ = NSUB <= 2;             // scores staged in LDS, written once per slab
+  constexpr int ZP = kBmSlab * NSUB + 1;
   __shared__ __align__(16) float sK[kChunk * KP];
+  __shared__ float s_z[kStageZ ? kBmRows * ZP : 1];
   __shared__ int s_maxls;
   const srswa_bm_score_args& a = p.a;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
   const int h = lane / 32, rl = lane % 32;
-  const int slab = blockIdx.x % p.nslab;
-  const int bt = blockIdx.x / p.nslab;
-  const int tile = p.ntiles - 1 - bt % p.ntiles;   // heaviest (last rows) first
+  // workgroups are dealt to the eight XCDs round-robin: an XCD takes every
+  // eighth row tile with all its slabs (a causal row tile reaches only the
+  // slabs before it, so dealing by slab left the XCDs of the last slabs idle),
+  // the tile fastest, so that its L2 serves a slab's keys to all of them
+  const int tpx = ceil_div(a.B * p.ntiles, 8);
+  const int bt = ((int)(blockIdx.x >> 3) % tpx) * 8 + (int)(blockIdx.x & 7);
+  const int slab = (int)(blockIdx.x >> 3) / tpx;
+  if (bt >= a.B * p.ntiles) return;
+  const int tile = bt % p.ntiles;
   const int b = bt / p.ntiles;
   const int row = tile * kBmRows + wave * 32 + rl;
   const bool row_ok = row < a.S;
@@ -723,9 +752,11 @@ __global__ __launch_bounds__(kBmThreads, 2) void bm_fwd_kernel(BmK p) {
     const int pos = a.pos[(int64_t)b * a.pos_sb + (int64_t)row * a.pos_st];
     ls = min(max(pos - a.local_window + 1, 0), a.S);
   }
+  const int wlo = wave_min_int(row_ok ? ls : INT_MAX);   // chunks below are scored whole by every row of the wave
+  const int whi = wave_max_int(ls);                      // chunks at or past hold no remote key of the wave
   if (tid == 0) s_maxls = 0;
   __syncthreads();
-  if (row_ok && h == 0) atomicMax(&s_maxls, ls);
+  if (lane == 0) atomicMax(&s_maxls, whi);
   __syncthreads();
   const int nchunks = ceil_div(s_maxls, kChunk);
   const int c_lo = slab * kBmSlab;
@@ -733,88 +764,122 @@ __global__ __launch_bounds__(kBmThreads, 2) void bm_fwd_kernel(BmK p) {
   const int blk_lo = c_lo * NSUB;
   const int blk_hi = slab == p.nslab - 1 ? a.nblk : min(a.nblk, (c_lo + kBmSlab) * NSUB);
 
-  float4 qf[D / 8];
-  {
-    const float* qrow = a.q + (int64_t)b * a.q_sb + (int64_t)(row_ok ? row : 0) * a.q_st;
-#pragma unroll
-    for (int m = 0; m < D / 8; ++m)
-      qf[m] = row_ok ? *reinterpret_cast<const float4*>(qrow + 8 * m + 4 * h) : make_float4(0.f, 0.f, 0.f, 0.f);
-  }
   float* zrow = a.z + (int64_t)b * a.z_sb + (int64_t)(row_ok ? row : 0) * a.z_st;
   int32_t* code = a.code + (int64_t)b * a.nblk * a.S + (row_ok ? row : 0);      // [b][blk][row]
   uint64_t* tm = a.tiemask + ((int64_t)b * a.S + (row_ok ? row : 0)) * a.nblk;   // [b][row][blk]
   const float* kg = a.k + (int64_t)b * a.k_sb;
-  constexpr int PR = D / 4;                       // 16-byte pieces per key row
-  constexpr int PPT = kChunk * PR / kBmThreads;   // per thread
-  float4 pre[PPT];
-  auto fetch = [&](int c) {
+  const float* qrow = a.q + (int64_t)b * a.q_sb + (int64_t)(row_ok ? row : 0) * a.q_st;
+  if (c_lo < c_hi) {
+    constexpr int PR = D / 4;                       // 16-byte pieces per key row
+    constexpr int PPT = kChunk * PR / kBmThreads;   // per thread
+    // a plain vector: as HIP's float4, a struct, the array was kept in scratch (960 us)
+    typedef float f32x4_t __attribute__((ext_vector_type(4)));
+    f32x4_t pre[PPT];
+    // keys past the last repeat it: they are never live (no branch here, or the
+    // loads would leave one by one, each waiting for the one before)
+    auto fetch = [&](int c) {
 #pragma unroll
-    for (int i = 0; i < PPT; ++i) {
-      const int pc = tid + kBmThreads * i;
-      const int j = c * kChunk + pc / PR, col = pc % PR;
-      pre[i] = j < a.S ? *reinterpret_cast<const float4*>(kg + (int64_t)j * a.k_st + 4 * col)
-                       : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-  };
-  if (c_lo < c_hi) fetch(c_lo);
-  for (int c = c_lo; c < c_hi; ++c) {
-    const int j0 = c * kChunk;
-    __syncthreads();
+      for (int i = 0; i < PPT; ++i) {
+        const int j = min(c * kChunk + i * (kBmThreads / PR) + tid / PR, a.S - 1);
+        pre[i] = *reinterpret_cast<const f32x4_t*>(kg + (int64_t)j * a.k_st + 4 * (tid % PR));
+      }
+    };
+    fetch(c_lo);
+    float4 qf[D / 8];
 #pragma unroll
-    for (int i = 0; i < PPT; ++i) {
-      const int pc = tid + kBmThreads * i;
-      *reinterpret_cast<float4*>(sK + (pc / PR) * KP + (pc % PR) * 4) = pre[i];
-    }
-    __syncthreads();
-    if (c + 1 < c_hi) fetch(c + 1);
-    const f32x16_t s0 = bm_tile<D>(sK, rl, qf, h);
-    const f32x16_t s1 = bm_tile<D>(sK, 32 + rl, qf, h);
+    for (int m = 0; m < D / 8; ++m) qf[m] = *reinterpret_cast<const float4*>(qrow + 8 * m + 4 * h);
+    for (int c = c_lo; c < c_hi; ++c) {
+      const int j0 = c * kChunk;
+      __syncthreads();                                // the previous chunk is consumed
 #pragma unroll
-    for (int sb = 0; sb < NSUB; ++sb) {
-      float mx = -INFINITY;
+      for (int i = 0; i < PPT; ++i) {
+        const int pc = tid + kBmThreads * i;
+        *reinterpret_cast<f32x4_t*>(sK + (pc / PR) * KP + 4 * (pc % PR)) = pre[i];
+      }
+      __syncthreads();
+      if (c + 1 < c_hi) fetch(c + 1);
+      const f32x16_t s0 = bm_tile<D>(sK, rl, qf, h);
+      const f32x16_t s1 = bm_tile<D>(sK, 32 + rl, qf, h);
+      // a lane's scores 16 half + r in one array; block sb of the chunk holds those with sub(i) == sb
+      auto val = [&](int i) __attribute__((always_inline)) { return i < 16 ? s0[i] : s1[i - 16]; };
+      auto sub = [](int i) __attribute__((always_inline)) {
+        return NSUB == 1 ? 0 : NSUB == 2 ? i / 16 : i / 8;
+      };
+      float mx[NSUB];
+      uint32_t tie = 0, grad = 0;                   // own bits
+      bool inside = j0 + kChunk <= wlo;
+      if (inside) {
+        // every key live: the largest score, clamped (the clamp is monotone)
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
+        for (int sb = 0; sb < NSUB; ++sb) mx[sb] = -kActClamp;
 #pragma unroll
-        for (int half = 0; half < 2; ++half) {
-          const int off = 32 * half + d_row(r, h);
-          if (off / BS == sb && j0 + off < ls) mx = fmaxf(mx, clamp_act(half ? s1[r] : s0[r]));
+        for (int i = 0; i < 32; ++i) mx[sub(i)] = fmaxf(mx[sub(i)], val(i));
+        bool in = true;
+#pragma unroll
+        for (int sb = 0; sb < NSUB; ++sb) {
+          mx[sb] = xor32_max(mx[sb]);
+          in = in && fabsf(mx[sb]) < kActClamp;
         }
-      mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
-      uint64_t tie = 0, grad = 0;                 // block-relative key bits
+        inside = __all(in);
+        if (inside) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
+          for (int i = 0; i < 32; ++i) tie |= val(i) == mx[sub(i)] ? 1u << i : 0u;
+          grad = tie;
+        }
+      }
+      if (!inside) {
+        const int lim = ls - j0 - 4 * h;            // score i is live when its key offset (less 4 h) is below
+        auto off = [](int i) __attribute__((always_inline)) { return 32 * (i / 16) + 8 * ((i % 16) >> 2) + (i & 3); };
 #pragma unroll
-        for (int half = 0; half < 2; ++half) {
-          const int off = 32 * half + d_row(r, h);
-          if (off / BS == sb && j0 + off < ls) {
-            const float raw = half ? s1[r] : s0[r];
-            const float cv = clamp_act(raw);
-            const uint64_t bit = 1ull << (off - sb * BS);
-            if (cv == mx) {
-              tie |= bit;
-              if (raw == cv) grad |= bit;
-            }
+        for (int sb = 0; sb < NSUB; ++sb) mx[sb] = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 32; ++i)
+          if (off(i) < lim) mx[sub(i)] = fmaxf(mx[sub(i)], clamp_act(val(i)));
+#pragma unroll
+        for (int sb = 0; sb < NSUB; ++sb) mx[sb] = xor32_max(mx[sb]);
+#pragma unroll
+        for (int i = 0; i < 32; ++i)
+          if (off(i) < lim && clamp_act(val(i)) == mx[sub(i)]) {
+            tie |= 1u << i;
+            if (clamp_act(val(i)) == val(i)) grad |= 1u << i;
+          }
+      }
+      const uint64_t tie64 = xor32_or(key_bits(tie, h)), grad64 = xor32_or(key_bits(grad, h));
+      if (row_ok && h == 0) {
+#pragma unroll
+        for (int sb = 0; sb < NSUB; ++sb) {
+          const int blk = c * NSUB + sb;
+          const uint64_t bm = BS == 64 ? ~0ull : (1ull << (BS % 64)) - 1ull;
+          const uint64_t tb = (tie64 >> (sb * BS % 64)) & bm, gb = (grad64 >> (sb * BS % 64)) & bm;
+          if (blk < a.nblk) {
+            const int ng = __popcll(gb);
+            int cd = kCodeNone;
+            if (ng > 0) cd = (int)__builtin_ctzll(gb) | (__popcll(tb) << 8) | (ng > 1 ? kCodeMulti : 0);
+            const float zv = mx[sb] == -INFINITY ? kScoreNeg : mx[sb];
+            if constexpr (kStageZ) s_z[(wave * 32 + rl) * ZP + blk - blk_lo] = zv;
+            else zrow[blk] = zv;
+            code[(int64_t)blk * a.S] = cd;
+            if (ng > 1) tm[blk] = gb;
           }
         }
-      tie |= shfl_xor_u64(tie, 32);
-      grad |= shfl_xor_u64(grad, 32);
-      const int blk = c * NSUB + sb;
-      if (row_ok && h == 0 && blk < a.nblk) {
-        const int ng = __popcll(grad);
-        int cd = kCodeNone;
-        if (ng > 0) cd = (int)__builtin_ctzll(grad) | (__popcll(tie) << 8) | (ng > 1 ? kCodeMulti : 0);
-        zrow[blk] = mx == -INFINITY ? kScoreNeg : mx;
-        code[(int64_t)blk * a.S] = cd;
-        if (ng > 1) tm[blk] = grad;
       }
     }
   }
-  // the slab's blocks after the last visited chunk hold no remote key of any row
-  if (row_ok && h == 0) {
-    for (int blk = max(c_hi > c_lo ? c_hi * NSUB : blk_lo, blk_lo); blk < blk_hi; ++blk) {
-      zrow[blk] = kScoreNeg;
-      code[(int64_t)blk * a.S] = kCodeNone;
+  const int done = max(c_hi > c_lo ? c_hi * NSUB : blk_lo, blk_lo);   // blocks at or past hold no remote key
+  if (row_ok && h == 0)
+    for (int blk = done; blk < blk_hi; ++blk) code[(int64_t)blk * a.S] = kCodeNone;
+  if constexpr (kStageZ) {
+    __syncthreads();
+    // 16 lanes per row: the slab's scores in runs of 64 bytes
+    for (int r = tid / 16; r < kBmRows; r += kBmThreads / 16) {
+      const int rw = tile * kBmRows + r;
+      if (rw >= a.S) break;
+      float* dst = a.z + (int64_t)b * a.z_sb + (int64_t)rw * a.z_st;
+      for (int blk = blk_lo + tid % 16; blk < blk_hi; blk += 16)
+        dst[blk] = blk < done ? s_z[r * ZP + blk - blk_lo] : kScoreNeg;
     }
+  } else if (row_ok && h == 0) {
+    for (int blk = done; blk < blk_hi; ++blk) zrow[blk] = kScoreNeg;
   }
 }
 
@@ -1235,7 +1300,7 @@ int bm_check(const srswa_bm_score_args* a, const char* what) {
 
 template <int D, int BS>
 void bm_launch_fwd(const BmK& k, hipStream_t st) {
-  const dim3 grid((unsigned)((int64_t)k.a.B * k.ntiles * k.nslab));
+  const dim3 grid((unsigned)(((int64_t)k.a.B * k.ntiles + 7) / 8 * 8 * k.nslab));
   hipLaunchKernelGGL((bm_fwd_kernel<D, BS>), grid, dim3(kBmThreads), 0, st, k);
 }
 
@@ -1283,7 +1348,7 @@ extern "C" int srswa_bm_score_fwd(const srswa_bm_score_args* a, void* stream) {
   k.a = *a;
   k.ntiles = ceil_div(a->S, kBmRows);
   k.nslab = std::max(1, ceil_div(ceil_div(a->S, kChunk), kBmSlab));
-  if ((int64_t)a->B * k.ntiles * k.nslab > 0x7fffffff) {
+  if (((int64_t)a->B * k.ntiles + 7) / 8 * 8 * k.nslab > 0x7fffffff) {
     set_error("block-max scores: grid too large");
     return SRSWA_UNSUPPORTED;
   }
