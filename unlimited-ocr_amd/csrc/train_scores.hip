@@ -52,8 +52,8 @@
 // v_mfma_f32_32x32x2_f32 as the inference block-max kernel, then per block the
 // clamped max, its tie and in-range masks), bm_bwd_dq (4 rows per wave, 16
 // waves per 64-row tile, the arg-max key rows of two blocks gathered
-// together) and bm_bwd_dk (four keys per wave, 16 lanes each, scanning the
-// block's codes in row order).  No atomics: every result is deterministic.
+// together) and bm_bwd_dk (a workgroup per block, four keys per wave, 16 lanes
+// each, scanning the block's codes in row order).  No atomics: every result is deterministic.
 #include <algorithm>
 #include <climits>
 #include <type_traits>
@@ -895,13 +895,19 @@ struct BmBK {
 __device__ __forceinline__ int bm_last_remote(int p, int LW, int BS) { return p - LW >= 0 ? (p - LW) / BS : -1; }
 
 // dq: 4 rows per wave, 16 waves per workgroup (64 rows); per group of 64
-// blocks the codes and weights g / n are staged in LDS (and the weights
-// stored block-major for bm_bwd_dk), then for each kBmBpi blocks up to the
-// tile's last remote one the wave's key rows of all of them are loaded
-// together (lanes over the head dims) and accumulated in block order.
+// blocks the codes and weights g / n are staged in LDS (and the weights stored
+// block-major for bm_bwd_dk).  Behind the router a row's gradient reaches the
+// few blocks of its entmax support and every other weight is exactly zero: a
+// wave whose rows weigh at most half of the group's blocks takes only those,
+// row by row, the key rows of kBmBatch of them loaded together (lanes over the
+// head dims); otherwise every block, the key rows of kBmBpi blocks and all
+// four rows together.  Both add in block order.  B = 2, S = 16384, 256 blocks,
+// the router's gradients: 157 us walking every block, 64 now; a gradient in
+// every block 276 and 291 us (361 when it took the first form too).
 constexpr int kBmRpw = 4;                               // rows per wave
 constexpr int kBmDqWaves = kTsRows / kBmRpw;
-constexpr int kBmBpi = 2;                               // blocks gathered together (divides kTsGroup)
+constexpr int kBmBatch = 8;                             // few blocks: key rows loaded together
+constexpr int kBmBpi = 2;                               // every block: blocks gathered together (divides kTsGroup)
 
 template <int D, int BS>
 __global__ __launch_bounds__(kBmDqWaves * kWave) void bm_bwd_dq_kernel(BmBK p) {
@@ -966,6 +972,61 @@ __global__ __launch_bounds__(kBmDqWaves * kWave) void bm_bwd_dq_kernel(BmBK p) {
       if (r < nr) wdst[(int64_t)c * a.S + r] = s_w[c * kTsPad + r];
     }
     const int cn = min(gn, trm - g0 + 1);
+    // several keys share a (row, block) gradient: each one in key order
+    auto several = [&](int r, int blk, float w) {
+      uint64_t m = a.tiemask[((int64_t)b * a.S + r0 + kBmRpw * wave + r) * a.nblk + blk];
+      while (m) {
+        const int off = __builtin_ctzll(m);
+        m &= m - 1;
+        const int j = blk * BS + off;
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) acc[r][e] = fmaf(w, kg[(int64_t)j * a.k_st + e], acc[r][e]);
+      }
+    };
+    // lane = block: the rows' weights, and which of them are not zero
+    float w_l[kBmRpw];
+    int cd_l[kBmRpw], total = 0;
+    uint64_t live[kBmRpw];
+#pragma unroll
+    for (int r = 0; r < kBmRpw; ++r) {
+      const int rr = kBmRpw * wave + r;
+      w_l[r] = lane < cn ? s_w[lane * kTsPad + rr] : 0.f;
+      cd_l[r] = lane < cn ? s_code[lane * kTsPad + rr] : 0;
+      live[r] = __ballot(w_l[r] != 0.f);
+      total += __popcll(live[r]);
+    }
+    if (total * 2 <= cn * kBmRpw) {
+#pragma unroll
+      for (int r = 0; r < kBmRpw; ++r) {
+        while (live[r]) {
+          float kv[kBmBatch][EPL], w[kBmBatch];
+          int cd[kBmBatch], blk[kBmBatch];
+#pragma unroll
+          for (int u = 0; u < kBmBatch; ++u) {
+            // past the last one: that one's row again, with no weight
+            const int c = live[r] ? (int)__builtin_ctzll(live[r]) : blk[u > 0 ? u - 1 : 0] - g0;
+            w[u] = live[r] ? __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w_l[r]), c)) : 0.f;
+            cd[u] = __builtin_amdgcn_readlane(cd_l[r], c);
+            blk[u] = g0 + c;
+            live[r] &= live[r] - 1;
+            const float* src = kg + (int64_t)(blk[u] * BS + (cd[u] & 0xff)) * a.k_st;
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) kv[u][e] = src[e];
+          }
+#pragma unroll
+          for (int u = 0; u < kBmBatch; ++u) {
+            if (w[u] == 0.f) continue;
+            if (!(cd[u] & kCodeMulti)) {
+#pragma unroll
+              for (int e = 0; e < EPL; ++e) acc[r][e] = fmaf(w[u], kv[u][e], acc[r][e]);
+            } else {
+              several(r, blk[u], w[u]);
+            }
+          }
+        }
+      }
+      continue;
+    }
     for (int c0 = 0; c0 < cn; c0 += kBmBpi) {               // c0 + kBmBpi <= 64: in the staged arrays
       float kv[kBmBpi][kBmRpw][EPL];
 #pragma unroll
@@ -987,7 +1048,6 @@ __global__ __launch_bounds__(kBmDqWaves * kWave) void bm_bwd_dq_kernel(BmBK p) {
       for (int u = 0; u < kBmBpi; ++u) {
         const int c = c0 + u;
         if (c >= cn) break;
-        const int blk = g0 + c;
 #pragma unroll
         for (int r = 0; r < kBmRpw; ++r) {
           const int rr = kBmRpw * wave + r;
@@ -998,15 +1058,7 @@ __global__ __launch_bounds__(kBmDqWaves * kWave) void bm_bwd_dq_kernel(BmBK p) {
 #pragma unroll
             for (int e = 0; e < EPL; ++e) acc[r][e] = fmaf(w, kv[u][r][e], acc[r][e]);
           } else {
-            // several keys share the gradient: each one in key order
-            uint64_t m = a.tiemask[((int64_t)b * a.S + r0 + rr) * a.nblk + blk];
-            while (m) {
-              const int off = __builtin_ctzll(m);
-              m &= m - 1;
-              const int j = blk * BS + off;
-#pragma unroll
-              for (int e = 0; e < EPL; ++e) acc[r][e] = fmaf(w, kg[(int64_t)j * a.k_st + e], acc[r][e]);
-            }
+            several(r, g0 + c, w);
           }
         }
       }
@@ -1023,30 +1075,33 @@ __global__ __launch_bounds__(kBmDqWaves * kWave) void bm_bwd_dq_kernel(BmBK p) {
   }
 }
 
-// dk: one wave per (sequence, block, four keys); lane group k (16 lanes)
-// owns key 4 w + k's D / 16 head dims per lane.  The block's codes and
-// weights are scanned 64 rows at a time in row order (the next batch loaded
-// while this one is taken); the rows whose gradient reaches a key are taken
-// one per lane group per step (four rows per load instruction).
+// dk: one workgroup per (sequence, block), a wave per four keys; lane group k
+// (16 lanes) of a wave owns its key k, D / 16 head dims per lane.  The block's
+// codes and weights pass through LDS once for all its waves, a row per thread
+// at a time (the next rows loaded while these are taken).  Every wave scans
+// them 64 rows at a time in row order and lists the rows whose gradient
+// reaches each of its keys; when a list may not hold 64 more, every lane group
+// adds up its key's list, kDkBatch query rows loaded together.  B = 2, S =
+// 16384, 256 blocks, a gradient in every block: 255 us, and 329 with each wave
+// reading the column for itself and adding the rows of every 64 as it met
+// them, one load latency after the other; the router's gradients 109 and 105.
+constexpr int kDkList = 96;     // list entries per key
+constexpr int kDkBatch = 4;
+
 template <int D, int BS>
-__global__ __launch_bounds__(256) void bm_bwd_dk_kernel(BmBK p) {
+__global__ __launch_bounds__(16 * BS) void bm_bwd_dk_kernel(BmBK p) {
   constexpr int DPL = D / 16;                    // head dims per lane
-  constexpr int QPB = BS / 4;                    // key quads per block
+  constexpr int NT = 16 * BS;                    // threads, and rows per batch
+  __shared__ int s_code[2][NT];
+  __shared__ float s_w[2][NT];
+  __shared__ __align__(16) int2 s_list[BS][kDkList];   // per key: (row, weight bits), rows ascending
   const srswa_bm_score_bwd_args& a = p.a;
-  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  // workgroups are dealt to the eight XCDs round-robin: consecutive logical
-  // ids (the quads of one block) are kept on one XCD so its L2 serves the
-  // block's code column to all of them
-  const int per_xcd = (int)(gridDim.x / 8);
-  const int64_t lid = (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  const int64_t gw = lid * 4 + wave;
+  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
   const int nblk_keys = min(a.nblk, ceil_div(a.S, BS));
-  if (gw >= (int64_t)a.B * nblk_keys * QPB) return;
-  const int quad = (int)(gw % QPB);
-  const int blk = (int)((gw / QPB) % nblk_keys);
-  const int b = (int)(gw / ((int64_t)QPB * nblk_keys));
+  const int blk = (int)blockIdx.x % nblk_keys;
+  const int b = (int)blockIdx.x / nblk_keys;
   const int kgrp = lane / 16, dl = lane % 16;
-  const int off0 = 4 * quad;                      // first key offset of the quad
+  const int off0 = 4 * wave;                      // first key offset of the wave's four
   const int my_key = off0 + kgrp;
   const int32_t* col = a.code + ((int64_t)b * a.nblk + blk) * a.S;
   const float* wcol = p.wT + ((int64_t)b * a.nblk + blk) * a.S;
@@ -1054,53 +1109,75 @@ __global__ __launch_bounds__(256) void bm_bwd_dk_kernel(BmBK p) {
   float acc[DPL];
 #pragma unroll
   for (int e = 0; e < DPL; ++e) acc[e] = 0.f;
-  int cd_n = lane < a.S ? col[lane] : kCodeNone;
-  float w_n = lane < a.S ? wcol[lane] : 0.f;
-  for (int i0 = 0; i0 < a.S; i0 += kWave) {
-    const int i = i0 + lane;
-    const int cd = cd_n;
-    const float w = w_n;
-    if (i + kWave < a.S) {
-      cd_n = col[i + kWave];
-      w_n = wcol[i + kWave];
-    } else {
-      cd_n = kCodeNone;
-      w_n = 0.f;
-    }
-    // which keys of the quad this row's gradient reaches (bit k)
-    uint32_t hit = 0;
-    if (w != 0.f) {
-      if (cd & kCodeMulti) {
-        const uint64_t m = a.tiemask[((int64_t)b * a.S + i) * a.nblk + blk];
-        hit = (uint32_t)((m >> off0) & 0xfu);
-      } else {
-        const int f = (cd & 0xff) - off0;
-        hit = (f >= 0 && f < 4) ? 1u << f : 0u;
+  int n[4] = {0, 0, 0, 0};                        // the lists' lengths (uniform)
+  auto add_lists = [&]() {
+    const int mine = kgrp == 0 ? n[0] : kgrp == 1 ? n[1] : kgrp == 2 ? n[2] : n[3];
+    const int most = max(max(n[0], n[1]), max(n[2], n[3]));
+    for (int t = 0; t < most; t += kDkBatch) {
+      int2 en[kDkBatch];
+      float4 qv[kDkBatch][DPL / 4];
+#pragma unroll
+      for (int u = 0; u < kDkBatch; ++u) {
+        en[u] = s_list[my_key][min(t + u, kDkList - 1)];
+        if (t + u >= mine) en[u] = make_int2(0, 0);       // row 0, added to nothing
       }
-    }
-    if (!__any(hit != 0)) continue;
-    uint64_t bal[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) bal[k] = __ballot((hit >> k) & 1u);
-    uint64_t mine = bal[kgrp];
-    // step n: every lane group takes its n-th row (rows in ascending order)
-    while (__any(mine != 0)) {
-      const int rsel = mine ? (int)__builtin_ctzll(mine) : 0;
-      const float wr = __shfl(w, rsel, kWave);
-      if (mine) {
-        mine &= mine - 1;
-        const float* qrow = qb + (int64_t)(i0 + rsel) * a.q_st;
+      for (int u = 0; u < kDkBatch; ++u)
 #pragma unroll
-        for (int e = 0; e < DPL; e += 4) {
-          const float4 qv = *reinterpret_cast<const float4*>(qrow + e);
-          acc[e] = fmaf(wr, qv.x, acc[e]);
-          acc[e + 1] = fmaf(wr, qv.y, acc[e + 1]);
-          acc[e + 2] = fmaf(wr, qv.z, acc[e + 2]);
-          acc[e + 3] = fmaf(wr, qv.w, acc[e + 3]);
+        for (int e = 0; e < DPL / 4; ++e)
+          qv[u][e] = *reinterpret_cast<const float4*>(qb + (int64_t)en[u].x * a.q_st + 4 * e);
+#pragma unroll
+      for (int u = 0; u < kDkBatch; ++u) {
+        const float w = __int_as_float(en[u].y);
+        if (t + u < mine) {
+#pragma unroll
+          for (int e = 0; e < DPL / 4; ++e) {
+            acc[4 * e] = fmaf(w, qv[u][e].x, acc[4 * e]);
+            acc[4 * e + 1] = fmaf(w, qv[u][e].y, acc[4 * e + 1]);
+            acc[4 * e + 2] = fmaf(w, qv[u][e].z, acc[4 * e + 2]);
+            acc[4 * e + 3] = fmaf(w, qv[u][e].w, acc[4 * e + 3]);
+          }
         }
       }
     }
+    n[0] = n[1] = n[2] = n[3] = 0;
+  };
+  int cd_n = tid < a.S ? col[tid] : kCodeNone;
+  float w_n = tid < a.S ? wcol[tid] : 0.f;
+  for (int r0 = 0, buf = 0; r0 < a.S; r0 += NT, buf ^= 1) {
+    s_code[buf][tid] = cd_n;
+    s_w[buf][tid] = w_n;
+    const int nx = r0 + NT + tid;
+    cd_n = nx < a.S ? col[nx] : kCodeNone;
+    w_n = nx < a.S ? wcol[nx] : 0.f;
+    __syncthreads();                              // the other buffer is free again past the next one
+    const int nrow = min(NT, a.S - r0);
+    for (int i0 = 0; i0 < nrow; i0 += kWave) {
+      const float w = s_w[buf][i0 + lane];
+      // which of the wave's keys this row's gradient reaches (bit k)
+      uint32_t hit = 0;
+      if (w != 0.f) {
+        const int cd = s_code[buf][i0 + lane];
+        if (cd & kCodeMulti) {
+          const uint64_t m = a.tiemask[((int64_t)b * a.S + r0 + i0 + lane) * a.nblk + blk];
+          hit = (uint32_t)((m >> off0) & 0xfu);
+        } else {
+          const int f = (cd & 0xff) - off0;
+          hit = (f >= 0 && f < 4) ? 1u << f : 0u;
+        }
+      }
+      if (!__any(hit != 0)) continue;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const bool on = (hit >> k) & 1u;
+        const uint64_t bal = __ballot(on);
+        if (on) s_list[off0 + k][n[k] + __popcll(bal & ((1ull << lane) - 1ull))] = make_int2(r0 + i0 + lane, __float_as_int(w));
+        n[k] += __popcll(bal);
+      }
+      if (max(max(n[0], n[1]), max(n[2], n[3])) > kDkList - kWave) add_lists();
+    }
   }
+  add_lists();
   const int j = blk * BS + my_key;
   if (j < a.S) {                                  // the last block may end past the keys
     float* dst = a.dk + (int64_t)b * a.dk_sb + (int64_t)j * a.dk_st + DPL * dl;
@@ -1310,10 +1387,8 @@ void bm_launch_bwd(const BmBK& k, hipStream_t st) {
   const int ntiles = (a.S + kTsRows - 1) / kTsRows;
   hipLaunchKernelGGL((bm_bwd_dq_kernel<D, BS>), dim3((unsigned)((int64_t)a.B * ntiles)), dim3(kBmDqWaves * kWave), 0,
                      st, k);
-  const int64_t waves = (int64_t)a.B * std::min(a.nblk, (a.S + BS - 1) / BS) * (BS / 4);
-  if (waves > 0)   // a multiple of 8 workgroups (the XCD deal), surplus ones exit at once
-    hipLaunchKernelGGL((bm_bwd_dk_kernel<D, BS>), dim3((unsigned)(((waves + 3) / 4 + 7) / 8 * 8)), dim3(256), 0,
-                       st, k);
+  const int64_t blocks = (int64_t)a.B * std::min(a.nblk, (a.S + BS - 1) / BS);
+  hipLaunchKernelGGL((bm_bwd_dk_kernel<D, BS>), dim3((unsigned)blocks), dim3(16 * BS), 0, st, k);
 }
 
 template <typename F>
