@@ -63,9 +63,10 @@ __global__ __launch_bounds__(256) void zero_words_kernel(uint32_t* w, int64_t n)
 }
 
 // One wavefront per (sequence, index head, query tile, slot), lane = row of
-// the tile.  When every live lane's block maps to the same chunk range (rows
-// of a tile sharing a selection), one lane sets the bits for the wave;
-// otherwise each lane sets its own.  Either way the bitmap gets the same bits.
+// the tile.  Of the lanes whose blocks map to the same chunk range one sets the
+// bits for all: the atomics of a tile's rows otherwise queue at the same few
+// words.  Rows that take 8 of their tile's 12 blocks each, T = 3001: 53 us with
+// one atomic per row and slot, 6.6 now (rows sharing a selection: 5).
 __global__ __launch_bounds__(256) void touch_kernel(BwdK p) {
   const srswa_bwd_args& a = p.a;
   const int lane = threadIdx.x % kWave;
@@ -98,16 +99,16 @@ __global__ __launch_bounds__(256) void touch_kernel(BwdK p) {
   const bool live = c1 >= c0;
   const uint64_t lm = __ballot(live);
   if (lm == 0ull) return;
-  const int first = __ffsll((long long)lm) - 1;
-  const int f0 = __shfl(c0, first, kWave), f1 = __shfl(c1, first, kWave);
-  const bool same = __all(!live || (c0 == f0 && c1 == f1));
-  uint32_t* base = p.touch + ((int64_t)b * a.HI + ih) * p.nchunk * p.twords + (tau >> 5);
-  if (same) {
-    if (lane == first)
-      for (int c = f0; c <= f1; ++c) atomicOr(base + (int64_t)c * p.twords, 1u << (tau & 31));
-  } else if (live) {
-    for (int c = c0; c <= c1; ++c) atomicOr(base + (int64_t)c * p.twords, 1u << (tau & 31));
+  bool leads = false;
+  for (uint64_t left = lm; left;) {
+    const int first = __builtin_ctzll(left);
+    const int f0 = __builtin_amdgcn_readlane(c0, first), f1 = __builtin_amdgcn_readlane(c1, first);
+    left &= ~__ballot(live && c0 == f0 && c1 == f1);
+    leads = leads || lane == first;
   }
+  uint32_t* base = p.touch + ((int64_t)b * a.HI + ih) * p.nchunk * p.twords + (tau >> 5);
+  if (leads)
+    for (int c = c0; c <= c1; ++c) atomicOr(base + (int64_t)c * p.twords, 1u << (tau & 31));
 }
 
 // -------------------------------------------------------------- 2. dQ
