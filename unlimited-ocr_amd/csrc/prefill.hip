@@ -73,9 +73,14 @@ struct FwdK {
 
 // ES: element bytes (2, or 4 for fp32, whose V^T operand is read as scalars:
 // a 4-float pad keeps the two lane halves' rows, 4 apart, on different banks)
-template <int D, int ES = 2> struct FwdLds {
+// The paged form gives up the V pitch without conflicts for 1 KB: with slot
+// biases and page ids a workgroup then stays within 40 KB, four per CU instead
+// of three.  Six requests of 70 to 1,900 biased rows: 164 -> 156 us bf16, 182
+// -> 166 fp8; four of 2,048: 141 -> 132.  (Contiguous, four per CU either way:
+// 0 to 1% slower with it.)
+template <int D, int ES = 2, bool PAGED = false> struct FwdLds {
   static constexpr int KP = D + 8;                  // K row pitch (elements): conflict-free row reads
-  static constexpr int VP = ES == 4 ? D + 4 : D + 16;   // V row pitch: conflict-free V^T reads
+  static constexpr int VP = ES == 4 ? D + 4 : PAGED ? D + 8 : D + 16;   // V row pitch: conflict-free V^T reads at + 16
   static constexpr int kOff = 0;
   static constexpr int vOff = kChunk * KP * ES;
   static constexpr int tileBytes = vOff + kChunk * VP * ES;
@@ -93,7 +98,7 @@ void fwd_kernel(FwdK p) {
   // a staged piece: 8 cache elements
   using Pre = std::conditional_t<FP8, uint2, Frag<T>>;
   using M = Mfma<T>;
-  using L = FwdLds<D, (int)sizeof(T)>;
+  using L = FwdLds<D, (int)sizeof(T), PAGED>;
   constexpr int KP = L::KP, VP = L::VP;
   constexpr int KS = D / 16;         // k-steps over the head dim
   constexpr int MT = D / 32;         // 32-row tiles of O^T
@@ -964,7 +969,7 @@ int plan_fwd_paged(const srswa_paged_fwd_args* a, FwdK& k, size_t& smem, size_t&
   const int64_t per_tile = (int64_t)kTileRows * a->S * (ceil_div(a->page_size, kChunk) + 1) +
                            ceil_div(f.local_window + kTileRows - 1, kChunk) + 1;
   const int umax = (int)std::min<int64_t>(nchunk, per_tile);
-  const size_t tile = a->D == 128 ? FwdLds<128>::tileBytes : FwdLds<64>::tileBytes;
+  const size_t tile = a->D == 128 ? FwdLds<128, 2, true>::tileBytes : FwdLds<64, 2, true>::tileBytes;
   const size_t setup = (3 * 64 + 4) * 4 + (size_t)k.nwords * 4;
   size_t n = std::max(tile, setup);
   k.chunks_off = (int)n;
