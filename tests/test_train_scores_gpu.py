@@ -261,6 +261,27 @@ def test_block_max_scores_fwd_bwd(dev, name):
         assert e <= F32_REL, (ez, eq, ek)
 
 
+@pytest.mark.parametrize("share", [0.01, 0.4, 0.6])
+@pytest.mark.parametrize("name", ["cfg5_like_bs64_lw512", "ragged_bs16_d64", "integer_ties_bs32",
+                                  "integer_ties_clamped_bs64"])
+def test_block_max_backward_few_gradients(dev, name, share):
+    """Most upstream gradients zero, as behind the router: both forms of dq (a
+    wave takes the first when its rows weigh at most half of a group's blocks;
+    ``share`` lies on either side) and short and long lists of dk, ties among them."""
+    from srswa import train_scores as TS
+    q, k, pos, nblk, bs, lw = _bm_case(name)
+    g = torch.Generator().manual_seed(21)
+    qr, kr = (x.double().requires_grad_() for x in (q, k))
+    zr = T.blockmax_scores(qr, kr, pos, nblk, bs, lw)
+    gz = torch.randn(zr.shape, generator=g) * (torch.rand(zr.shape, generator=g) < share)
+    zr.backward(gz.double())
+    qd, kd = (x.to(dev).requires_grad_() for x in (q, k))
+    TS.block_max_scores(qd, kd, pos.to(dev), nblk, bs, lw).backward(gz.to(dev))
+    eq, ek = _rel(qd.grad, qr.grad), _rel(kd.grad, kr.grad)
+    report(f"[err] block-max backward {name}, {share:.0%} of the gradients: dq {eq:.3e}, dk {ek:.3e} (bar {F32_REL})")
+    assert max(eq, ek) <= F32_REL
+
+
 def test_block_max_scores_deterministic(dev):
     from srswa import train_scores as TS
     q, k, pos, nblk, bs, lw = _bm_case("integer_ties_bs32")
