@@ -8,6 +8,8 @@ replays; every replay must equal the eager result bit for bit.
 * the DASH serving decode step: per-page summary tail refresh -> summary
   scores -> router -> paged decode;
 * srswa_gather_decode_noalloc (split-K records in the library's static array);
+* the gather-attention forward of a launch that is split over idle CUs, with
+  larger calls on the same stream between capture and replay;
 * the gather-KL forward (row-sparse, tile kernels forked onto the caller's
   second stream and joined back) and its backward.
 
@@ -26,7 +28,7 @@ REPLAYS = 3
 
 def _capture(fn, warm=2):
     """(graph, outputs of the captured call) with fn run eagerly on the side
-    stream first (allocations of per-stream scratch, first-use set-up)."""
+    stream first (first-use set-up)."""
     s = torch.cuda.Stream()
     s.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(s):
@@ -121,6 +123,45 @@ def test_graph_noalloc_decode(dev):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, o_ref) and torch.equal(lse, l_ref)
+
+
+def test_graph_split_forward_after_larger_calls(dev):
+    """320 tiles, two parts each, captured; then eager calls with more scratch
+    on the capture stream, and tensors in whatever they freed, before each replay:
+    the graph's part records must be its own memory."""
+    from srswa import ops
+    g0 = torch.Generator().manual_seed(12)
+    B, T, H, D, S = 1, 2048, 10, 128, 4
+    q, k, v = (torch.randn(B, T, H, D, generator=g0).to(torch.bfloat16).to(dev) for _ in range(3))
+    idx = torch.randint(-1, T // 64, (B, 1, T, S), generator=g0).to(torch.int32).to(dev)
+    kw = dict(block_size=64, local_window=512, scale=D ** -0.5)
+    call = lambda: ops.gather_fwd(q, k, v, idx, **kw)
+    gen = torch.Generator(device=dev).manual_seed(13)
+    inputs = [torch.randn(q.shape, device=dev, generator=gen).to(q.dtype) for _ in range(REPLAYS)]
+    eager = []
+    for qi in inputs:
+        q.copy_(qi)
+        eager.append(tuple(t.clone() for t in call()))
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        call()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        out, lse = call()
+    torch.cuda.synchronize()
+    for qi, (o_ref, l_ref) in zip(inputs, eager):
+        q.copy_(qi)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(s):
+            ops.gather_bwd(q, k, v, o_ref, l_ref, o_ref, idx, **kw)
+            others = [torch.full((1 << 20,), 7.0, device=dev) for _ in range(16)]
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, o_ref) and torch.equal(lse, l_ref)
+        assert all(bool((t == 7.0).all()) for t in others)
 
 
 def test_graph_gather_kl_fwd_bwd_with_side_stream(dev):

@@ -706,20 +706,11 @@ def ptr(t) -> int | None:
     return None if t is None else t.data_ptr()
 
 
-_scratch_cache: dict = {}
-
-
-def _stream_key(device: torch.device):
-    return (device.index, stream_ptr(device))
-
-
 def scratch(device: torch.device, nbytes: int) -> torch.Tensor | None:
-    """Device scratch (no content requirement), cached per (device, stream)."""
-    if nbytes <= 0:
-        return None
-    key = _stream_key(device)
-    buf = _scratch_cache.get(key)
-    if buf is None or buf.numel() < nbytes:
-        buf = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
-        _scratch_cache[key] = buf
-    return buf
+    """Device scratch (no content requirement) of one call.  Nothing is kept
+    between calls: two host threads on one stream would write the same records
+    between each other's launches, and a captured graph would replay into a
+    buffer that a later, larger call had replaced.  The caching allocator hands
+    the same memory out again in stream order, and from the graph's pool under
+    capture."""
+    return torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes > 0 else None

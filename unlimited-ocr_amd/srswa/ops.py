@@ -422,7 +422,7 @@ def gather_fwd_paged(q, k_cache, v_cache, topk_idx, blk_bias, block_table, cu_se
     a.kv_fp8 = kv8
     # the split's workspace (0 bytes for a launch that fills the GPU)
     nws = _lib.lib().srswa_gather_fwd_paged_workspace(ctypes.byref(a))
-    ws = torch.empty(nws, dtype=torch.uint8, device=q.device) if nws else None
+    ws = _lib.scratch(q.device, nws)
     _lib.check(_lib.lib().srswa_gather_fwd_paged_ws(ctypes.byref(a), _lib.ptr(ws), nws, _lib.stream_ptr(q.device)),
                "srswa_gather_fwd_paged_ws")
     return out
@@ -673,7 +673,7 @@ def gather_fwd(q, k, v, block_indices, *, block_size, local_window, scale, seg=N
     a.block_size, a.local_window = int(block_size), max(1, int(local_window))
     a.scale = float(scale)
     a.dtype = _lib.dtype_code(q.dtype)
-    # the tail split's workspace (0 bytes when the launch's last round is full)
+    # the split's workspace (0 bytes for a launch that fills the GPU)
     nws = _lib.lib().srswa_gather_fwd_workspace(ctypes.byref(a)) if tail_split else 0
     ws = _lib.scratch(q.device, nws)
     _lib.check(_lib.lib().srswa_gather_fwd_ws(ctypes.byref(a), _lib.ptr(ws), nws, _lib.stream_ptr(q.device)),
