@@ -1075,6 +1075,13 @@ __global__ __launch_bounds__(kBmDqWaves * kWave) void bm_bwd_dq_kernel(BmBK p) {
   }
 }
 
+// the wave's LDS writes before its later reads by other lanes, and the other way round
+__device__ __forceinline__ void wave_sync_lds() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // dk: one workgroup per (sequence, block), a wave per four keys; lane group k
 // (16 lanes) of a wave owns its key k, D / 16 head dims per lane.  The block's
 // codes and weights pass through LDS once for all its waves, a row per thread
@@ -1113,6 +1120,7 @@ __global__ __launch_bounds__(16 * BS) void bm_bwd_dk_kernel(BmBK p) {
   auto add_lists = [&]() {
     const int mine = kgrp == 0 ? n[0] : kgrp == 1 ? n[1] : kgrp == 2 ? n[2] : n[3];
     const int most = max(max(n[0], n[1]), max(n[2], n[3]));
+    wave_sync_lds();                             // entries come from any lane of the wave
     for (int t = 0; t < most; t += kDkBatch) {
       int2 en[kDkBatch];
       float4 qv[kDkBatch][DPL / 4];
@@ -1141,6 +1149,7 @@ __global__ __launch_bounds__(16 * BS) void bm_bwd_dk_kernel(BmBK p) {
       }
     }
     n[0] = n[1] = n[2] = n[3] = 0;
+    wave_sync_lds();                             // read before the next entries overwrite them
   };
   int cd_n = tid < a.S ? col[tid] : kCodeNone;
   float w_n = tid < a.S ? wcol[tid] : 0.f;
