@@ -3,9 +3,10 @@ refuse.  No kernel is launched (CPU-only)."""
 
 import weakref
 
+import pytest
 import torch
 
-from srswa import _lib
+from srswa import _lib, dash_train
 
 CPU = torch.device("cpu")
 
@@ -21,3 +22,32 @@ def test_scratch_belongs_to_one_call(monkeypatch):
     del a
     assert kept() is None
     assert _lib.scratch(CPU, 0) is None
+
+
+def test_stream_of_a_host_device_is_refused(monkeypatch):
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda idx: 0, raising=False)
+    for device in (CPU, torch.device("meta")):
+        with pytest.raises(ValueError, match="Expected a cuda device"):
+            _lib.stream_ptr(device)
+    assert _lib.stream_ptr(torch.device("cuda")) == 0 and _lib.stream_ptr(torch.device("cuda", 0)) == 0
+
+
+def test_host_tensors_reach_no_launch(monkeypatch):
+    """The launchers without a check of their own refuse host tensors through
+    the stream they ask for, before the library is called."""
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda idx: 0, raising=False)
+    launched = []
+
+    class Lib:
+        def __getattr__(self, name):
+            return lambda *a: launched.append(name) or 0
+
+    monkeypatch.setattr(_lib, "lib", Lib)
+    prior, cand = torch.rand(4, 8), torch.ones(4, 8, dtype=torch.bool)
+    with pytest.raises(ValueError, match="Expected a cuda device"):
+        dash_train.select_forward(prior, cand, 2, 1e-4, 1.0)
+    with pytest.raises(ValueError, match="Expected a cuda device"):
+        dash_train.route_backward(prior, prior, cand, 1.0)
+    assert launched == []

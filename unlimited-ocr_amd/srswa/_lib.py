@@ -695,9 +695,12 @@ def dtype_code(dt: torch.dtype) -> int:
 
 def stream_ptr(device: torch.device) -> int:
     """Handle of the current stream of ``device``, without building the
-    ``torch.cuda.Stream`` object around it (every call asks for it, most of
-    them twice).  With the strides read as one tuple per tensor, a call of one
-    kernel went from 23.9 to 18.6 us on the host."""
+    ``torch.cuda.Stream`` object around it (every call asks for it).  With the
+    strides read as one tuple per tensor, a call of one kernel went from 23.9 to
+    18.6 us on the host.  Refuses any other device, as that object does: most
+    launchers have no other check that their tensors are on the GPU."""
+    if device.type != "cuda":
+        raise ValueError(f"Expected a cuda device, but got: {device}")
     idx = device.index
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if idx is None else idx)
 
