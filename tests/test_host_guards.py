@@ -6,7 +6,7 @@ import weakref
 import pytest
 import torch
 
-from srswa import _lib, dash_train
+from srswa import _lib, dash_train, ops
 
 CPU = torch.device("cpu")
 
@@ -51,3 +51,14 @@ def test_host_tensors_reach_no_launch(monkeypatch):
     with pytest.raises(ValueError, match="Expected a cuda device"):
         dash_train.route_backward(prior, prior, cand, 1.0)
     assert launched == []
+
+
+def test_backward_bias_must_cover_the_query_rows(monkeypatch):
+    """A bias (and ids) of fewer rows than the queries would be read past its end."""
+    monkeypatch.setattr(ops, "_require_cuda", lambda *ts: None)
+    B, T, H, D, S = 1, 64, 2, 64, 3
+    q, lse = torch.zeros(B, T, H, D), torch.zeros(B, T, H)
+    for rows in (T // 2, T + 1):
+        ids, bias = torch.zeros(B, 1, rows, S, dtype=torch.int32), torch.zeros(B, rows, S)
+        with pytest.raises(RuntimeError, match="expand"):
+            ops.gather_bwd(q, q, q, q, lse, q, ids, block_size=64, local_window=64, scale=1.0, bias=bias)

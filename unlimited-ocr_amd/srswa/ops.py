@@ -694,7 +694,7 @@ def gather_bwd(q, k, v, o, lse, do, block_indices, *, block_size, local_window, 
     if bias is not None:
         if bias.dim() == 3:
             bias = bias.unsqueeze(1)
-        bias = _as(bias, torch.float32, idx.shape)
+        bias = _as(bias, torch.float32, (B, HI, T, S))
     if seg is not None:
         seg = _i32(seg).contiguous()
     if do.stride(-1) != 1:
