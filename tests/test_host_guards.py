@@ -1,6 +1,8 @@
 """Host-side guarantees of the launch helpers: what they allocate, keep and
 refuse.  No kernel is launched (CPU-only)."""
 
+import ctypes
+import warnings
 import weakref
 
 import pytest
@@ -62,3 +64,41 @@ def test_backward_bias_must_cover_the_query_rows(monkeypatch):
         ids, bias = torch.zeros(B, 1, rows, S, dtype=torch.int32), torch.zeros(B, rows, S)
         with pytest.raises(RuntimeError, match="expand"):
             ops.gather_bwd(q, q, q, q, lse, q, ids, block_size=64, local_window=64, scale=1.0, bias=bias)
+
+
+@pytest.mark.parametrize("shape", [(5,), (1, 5), (3, 5), (3, 1)])
+def test_sample_starts_broadcast(shape):
+    """Positions of one row, or of one column, stand for all of them, without
+    torch's warning of a resized output."""
+    pos = torch.arange(15).view(3, 5)[:shape[0] if len(shape) == 2 else 1, :shape[-1]].reshape(shape)
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        seg = ops._seg_from_positions(pos, 5, 9, CPU)
+    assert seg.dtype == torch.int32
+    assert torch.equal(seg.long(), torch.arange(4, 9)[None] - pos)
+
+
+@pytest.mark.parametrize("rows", [(4,), (1, 4), (3, 4)])
+def test_forward_reads_sample_starts_of_every_sequence(monkeypatch, rows):
+    """The kernel reads seg [B, T] by its strides: one row given for three
+    sequences must not be read past its end."""
+    seen = []
+
+    class Lib:
+        def srswa_gather_fwd_workspace(self, a):
+            return 0
+
+        def srswa_gather_fwd_ws(self, a, ws, nws, stream):
+            f = a._obj
+            raw = (ctypes.c_int32 * (2 * f.seg_sb + f.T)).from_address(f.seg)
+            seen.append(torch.tensor([[raw[b * f.seg_sb + t] for t in range(f.T)] for b in range(f.B)]))
+            return 0
+
+    monkeypatch.setattr(ops, "_require_cuda", lambda *ts: None)
+    monkeypatch.setattr(_lib, "stream_ptr", lambda device: 0)
+    monkeypatch.setattr(_lib, "lib", Lib)
+    B, T, H, D = 3, 4, 2, 64
+    q = torch.zeros(B, T, H, D)
+    seg = torch.arange(torch.Size(rows).numel()).view(rows)
+    ops.gather_fwd(q, q, q, torch.zeros(B, 1, T, 2, dtype=torch.int32), block_size=64, local_window=64, scale=1.0, seg=seg)
+    assert torch.equal(seen[0].long(), seg.expand(B, T))

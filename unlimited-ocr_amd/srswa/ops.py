@@ -622,7 +622,8 @@ def _seg_from_positions(position_ids, T, Sk, device):
         return None
     qi = torch.arange(Sk - T, Sk, device=device, dtype=torch.int64)
     pos = position_ids.to(device=device, dtype=torch.int64)
-    return torch.sub(qi, pos, out=torch.empty(pos.shape, dtype=torch.int32, device=device))   # narrowed as it is stored
+    out = torch.empty(torch.broadcast_shapes((1, T), pos.shape), dtype=torch.int32, device=device)
+    return torch.sub(qi, pos, out=out)                                   # narrowed as it is stored
 
 
 def gather_fwd(q, k, v, block_indices, *, block_size, local_window, scale, seg=None, bias=None,
@@ -631,7 +632,7 @@ def gather_fwd(q, k, v, block_indices, *, block_size, local_window, scale, seg=N
 
     q [B, T, HQ, D]; k, v [B, Sk, HKV, D] (Sk >= T, queries are the last T
     keys); block_indices [B, HI, T, S] (-1 pad); seg [B, T] int sample starts
-    (None = 0); bias [B, T, S] or [B, HI, T, S] per-slot bias on remote keys.
+    (or [1, T] for every sequence; None = 0); bias [B, T, S] or [B, HI, T, S] per-slot bias on remote keys.
     tail_split=False runs every tile as one workgroup (no workspace).
     Returns (o [B, T, HQ, D], lse [B, T, HQ] fp32 or None)."""
     _require_cuda(q, k, v, block_indices, seg, bias)
@@ -653,7 +654,7 @@ def gather_fwd(q, k, v, block_indices, *, block_size, local_window, scale, seg=N
             bias = bias.unsqueeze(1)
         bias = _as(bias, torch.float32, idx.shape)
     if seg is not None:
-        seg = _i32(seg).contiguous()
+        seg = _as(seg, torch.int32, (B, T))
     if out is None:
         out = torch.empty(B, T, HQ, D, dtype=q.dtype, device=q.device)
     lse = torch.empty(B, T, HQ, dtype=torch.float32, device=q.device) if need_lse else None
@@ -696,7 +697,7 @@ def gather_bwd(q, k, v, o, lse, do, block_indices, *, block_size, local_window, 
             bias = bias.unsqueeze(1)
         bias = _as(bias, torch.float32, (B, HI, T, S))
     if seg is not None:
-        seg = _i32(seg).contiguous()
+        seg = _as(seg, torch.int32, (B, T))
     if do.stride(-1) != 1:
         do = do.contiguous()
     dq = torch.empty(B, T, HQ, D, dtype=q.dtype, device=q.device)
