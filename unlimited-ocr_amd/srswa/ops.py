@@ -623,7 +623,7 @@ def _seg_from_positions(position_ids, T, Sk, device):
     qi = torch.arange(Sk - T, Sk, device=device, dtype=torch.int64)
     pos = position_ids.to(device=device, dtype=torch.int64)
     out = torch.empty(torch.broadcast_shapes((1, T), pos.shape), dtype=torch.int32, device=device)
-    return torch.sub(qi, pos, out=out)                                   # narrowed as it is stored
+    return torch.sub(qi[None], pos, out=out)                             # narrowed as it is stored
 
 
 def gather_fwd(q, k, v, block_indices, *, block_size, local_window, scale, seg=None, bias=None,
