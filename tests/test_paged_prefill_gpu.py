@@ -157,3 +157,52 @@ def test_split_launch_matches_whole_tiles(dev, monkeypatch, max_q, parts, kv):
     assert ((split - whole).abs() <= 2.0 ** -8 * vc.float().abs().max() + ulp).all()
     if parts == 1:
         assert torch.equal(split, whole)
+
+
+def _request_case(dev, seed, q_lens, ctx, *, H, HKV, D, page, K, dtype, kv=None, bias=True):
+    """Requests over pages dealt in random order, every row its own selection."""
+    g = torch.Generator(device=dev).manual_seed(seed)
+    seq = [a + b for a, b in zip(q_lens, ctx)]
+    nb, total = -(-max(seq) // page), sum(q_lens)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev).to(dtype)
+    kc, vc = (rnd(len(seq) * nb, page, HKV, D).to(kv or dtype) for _ in range(2))
+    return dict(q=rnd(total, H, D), k=kc, v=vc, page=page, HKV=HKV, q_lens=q_lens, ctx=ctx,
+                bt=torch.randperm(len(seq) * nb, generator=g, device=dev).view(len(seq), nb).to(torch.int32),
+                ids=torch.randint(-1, nb, (HKV, total, K), generator=g, device=dev).to(torch.int32),
+                bias=torch.randn(HKV, total, K, generator=g, device=dev) if bias else None)
+
+
+def _attend(c, pieces=None):
+    """The requests' rows in one launch, or ``pieces`` [(request, first row, rows)] as its requests."""
+    dev, starts = c["q"].device, [sum(c["q_lens"][:i]) for i in range(len(c["q_lens"]))]
+    pieces = pieces or [(r, 0, n) for r, n in enumerate(c["q_lens"])]
+    rows = torch.cat([torch.arange(starts[r] + t, starts[r] + t + n) for r, t, n in pieces]).to(dev)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)
+    q = c["q"][rows]
+    out = torch.zeros_like(q)
+    U.dash_sparse_attn(q, c["k"], c["v"], c["ids"][:, rows].contiguous(),
+                       None if c["bias"] is None else c["bias"][:, rows].contiguous(),
+                       c["bt"][[r for r, _, _ in pieces]].contiguous(),
+                       i32([0] + [n for _, _, n in pieces]).cumsum(0).to(torch.int32),
+                       i32([c["ctx"][r] + c["q_lens"][r] for r, _, _ in pieces]), i32([c["ctx"][r] + t for r, t, _ in pieces]),
+                       max(n for _, _, n in pieces), c["HKV"], q.shape[-1] ** -0.5, out, local_blocks=2,
+                       sparse_block_size=c["page"])
+    return out
+
+
+@pytest.mark.parametrize("D,K,page,ctx,kv", [(128, 8, 64, 20000, None), (128, 8, 64, 20000, torch.float8_e4m3fn),
+                                             (128, 12, 16, 5000, None), (64, 39, 64, 29000, None),
+                                             (64, 39, 64, 29000, torch.float8_e5m2)])
+def test_more_rounds_than_one_match_short_launches(dev, monkeypatch, D, K, page, ctx, kv):
+    """784 tiles of one request, more than three workgroups per CU: a layout that
+    holds four takes the narrower V pitch.  Launches of 400 and 384 of the same
+    tiles take the other; both visit the same chunks in the same order, so
+    their rows agree to the last bit.  (Without the split, which rounds otherwise.)"""
+    from srswa import _lib
+    monkeypatch.setattr(_lib.lib(), "srswa_gather_fwd_paged_workspace", lambda a: 0)
+    c = _request_case(dev, D + K, [49 * 64 - 5], [ctx], H=16, HKV=16, D=D, page=page, K=K, dtype=torch.bfloat16, kv=kv)
+    whole = _attend(c)
+    first = _attend(c, [(0, 0, 25 * 64)])
+    second = _attend(c, [(0, 25 * 64, 24 * 64 - 5)])
+    assert torch.isfinite(whole.float()).all()
+    assert torch.equal(whole, torch.cat([first, second]))

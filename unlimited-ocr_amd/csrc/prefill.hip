@@ -25,7 +25,7 @@
 // selected blocks of all 64 rows: bitmap + prefix popcount), so a tile whose
 // rows share their selection visits |selected| + |window| chunks once.
 // Per chunk:
-//   * K (row pitch D+8) and V (row pitch D+16) are staged in LDS from
+//   * K (row pitch D+8) and V (row pitch D+16, or D+8: FwdLds) are staged in LDS from
 //     registers fetched one chunk ahead;
 //   * S^T = K Q^T on v_mfma_f32_32x32x16_{bf16,f16}: every lane owns one
 //     query row and 32 of the chunk's keys;
@@ -63,24 +63,24 @@ struct FwdK {
   const int32_t* bt;
   int64_t bt_sr, k_pst, v_pst;
   int kv8;                     // FP8: the caches' fp8 format (srswa_dtype)
-  // tail split: the last ntail logical tiles run as nsplit workgroups each, part
-  // p taking chunks [U p / nsplit, U (p + 1) / nsplit) of the tile's plan and
-  // writing an unnormalised record (O fp32 [64][D], then m, l per row) that
-  // fwd_merge_kernel combines.  The whole tiles come first in dispatch order.
+  bool narrow;                 // paged: the shorter V pitch (FwdLds)
+  // split: the last ntail logical tiles (paged: all or none) run as nsplit
+  // workgroups each, part p taking chunks [U p / nsplit, U (p + 1) / nsplit) of
+  // the tile's plan and writing an unnormalised record (O fp32 [64][D], then m, l
+  // per row) that fwd_merge_kernel combines.  Whole tiles come first in dispatch order.
   int nsplit, ntail, per_xcd_p;
   float* part;                 // [ntail * nsplit][64 * D + 128]
 };
 
 // ES: element bytes (2, or 4 for fp32, whose V^T operand is read as scalars:
 // a 4-float pad keeps the two lane halves' rows, 4 apart, on different banks)
-// The paged form gives up the V pitch without conflicts for 1 KB: with slot
-// biases and page ids a workgroup then stays within 40 KB, four per CU instead
-// of three.  Six requests of 70 to 1,900 biased rows: 164 -> 156 us bf16, 182
-// -> 166 fp8; four of 2,048: 141 -> 132.  (Contiguous, four per CU either way:
-// 0 to 1% slower with it.)
-template <int D, int ES = 2, bool PAGED = false> struct FwdLds {
+// NARROW gives up the V pitch without conflicts for 1 KB: the paged form with
+// slot biases and page ids can then stay within 40 KB, four workgroups per CU
+// instead of three.  The plan takes it only where that lets the launch run in
+// fewer rounds (plan_fwd_paged).
+template <int D, int ES = 2, bool NARROW = false> struct FwdLds {
   static constexpr int KP = D + 8;                  // K row pitch (elements): conflict-free row reads
-  static constexpr int VP = ES == 4 ? D + 4 : PAGED ? D + 8 : D + 16;   // V row pitch: conflict-free V^T reads at + 16
+  static constexpr int VP = ES == 4 ? D + 4 : NARROW ? D + 8 : D + 16;   // V row pitch: conflict-free V^T reads at + 16
   static constexpr int kOff = 0;
   static constexpr int vOff = kChunk * KP * ES;
   static constexpr int tileBytes = vOff + kChunk * VP * ES;
@@ -88,7 +88,7 @@ template <int D, int ES = 2, bool PAGED = false> struct FwdLds {
 
 // Two waves per SIMD; the fp32 form at D = 128 (twice the operand registers)
 // one, with the accumulators in the second register file.
-template <typename T, int D, bool PAGED, bool FP8 = false>
+template <typename T, int D, bool PAGED, bool FP8 = false, bool NARROW = false>
 __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(std::is_same<T, float>::value && D == 128 ? 1 : 2)))
 void fwd_kernel(FwdK p) {
   static_assert(!FP8 || PAGED, "fp8 caches: the paged form");
@@ -98,7 +98,7 @@ void fwd_kernel(FwdK p) {
   // a staged piece: 8 cache elements
   using Pre = std::conditional_t<FP8, uint2, Frag<T>>;
   using M = Mfma<T>;
-  using L = FwdLds<D, (int)sizeof(T), PAGED>;
+  using L = FwdLds<D, (int)sizeof(T), NARROW>;
   constexpr int KP = L::KP, VP = L::VP;
   constexpr int KS = D / 16;         // k-steps over the head dim
   constexpr int MT = D / 32;         // 32-row tiles of O^T
@@ -722,12 +722,12 @@ int check_fwd(const srswa_fwd_args* a) {
   return SRSWA_OK;
 }
 
-template <typename T, int D, bool PAGED, bool FP8 = false>
+template <typename T, int D, bool PAGED, bool FP8 = false, bool NARROW = false>
 int launch_fwd(const FwdK& k, size_t smem, hipStream_t st) {
   static LdsGrant granted;
-  if (!ensure_dynamic_lds(&fwd_kernel<T, D, PAGED, FP8>, smem, &granted)) return SRSWA_UNSUPPORTED;
+  if (!ensure_dynamic_lds(&fwd_kernel<T, D, PAGED, FP8, NARROW>, smem, &granted)) return SRSWA_UNSUPPORTED;
   const unsigned grid = PAGED ? (unsigned)(k.nlogical * k.nsplit) : (unsigned)(8 * k.per_xcd + 8 * k.per_xcd_p);
-  hipLaunchKernelGGL((fwd_kernel<T, D, PAGED, FP8>), dim3(grid), dim3(128), smem, st, k);
+  hipLaunchKernelGGL((fwd_kernel<T, D, PAGED, FP8, NARROW>), dim3(grid), dim3(128), smem, st, k);
   if (k.ntail > 0) {
     const dim3 mg((unsigned)(4 * k.ntail));
     if (k.nsplit == 8) hipLaunchKernelGGL((fwd_merge_kernel<T, D, PAGED, 8>), mg, dim3(256), 0, st, k);
@@ -740,6 +740,13 @@ int launch_fwd(const FwdK& k, size_t smem, hipStream_t st) {
     return SRSWA_LAUNCH;
   }
   return SRSWA_OK;
+}
+
+template <typename T, bool FP8>
+int launch_fwd_paged(const FwdK& k, size_t smem, hipStream_t st) {
+  if (k.a.D == 128)
+    return k.narrow ? launch_fwd<T, 128, true, FP8, true>(k, smem, st) : launch_fwd<T, 128, true, FP8>(k, smem, st);
+  return k.narrow ? launch_fwd<T, 64, true, FP8, true>(k, smem, st) : launch_fwd<T, 64, true, FP8>(k, smem, st);
 }
 
 }  // namespace
@@ -969,29 +976,47 @@ int plan_fwd_paged(const srswa_paged_fwd_args* a, FwdK& k, size_t& smem, size_t&
   const int64_t per_tile = (int64_t)kTileRows * a->S * (ceil_div(a->page_size, kChunk) + 1) +
                            ceil_div(f.local_window + kTileRows - 1, kChunk) + 1;
   const int umax = (int)std::min<int64_t>(nchunk, per_tile);
-  const size_t tile = a->D == 128 ? FwdLds<128, 2, true>::tileBytes : FwdLds<64, 2, true>::tileBytes;
   const size_t setup = (3 * 64 + 4) * 4 + (size_t)k.nwords * 4;
-  size_t n = std::max(tile, setup);
-  k.chunks_off = (int)n;
-  n += ((size_t)umax * 2 + 15) / 16 * 16;
-  k.sid_off = (int)n;
-  n += (size_t)64 * k.SP * 4 * (a->bias ? 2 : 1);
-  // page ids of the visited chunks in the LDS left below 40 KB (four
-  // workgroups per CU), or below 52 KB when the rest already exceeds it
-  k.ppc = a->page_size >= kChunk ? 1 : 4;
-  k.pages_off = (int)((n + 15) / 16 * 16);
-  const size_t budget = k.pages_off <= 40 * 1024 - 64 ? 40 * 1024 : 52 * 1024;
-  k.page_cap = (int)std::min<int64_t>(umax, k.pages_off < (int)budget ? (budget - k.pages_off) / (4 * k.ppc) : 0);
-  n = k.pages_off + (size_t)k.page_cap * 4 * k.ppc;
-  smem = (n + 15) / 16 * 16;
+  const int cus = device_cu_count();
+  // LDS of the layout with `tile` bytes of K and V, and the workgroups a CU holds with it
+  auto layout = [&](size_t tile) {
+    size_t n = std::max(tile, setup);
+    k.chunks_off = (int)n;
+    n += ((size_t)umax * 2 + 15) / 16 * 16;
+    k.sid_off = (int)n;
+    n += (size_t)64 * k.SP * 4 * (a->bias ? 2 : 1);
+    // page ids of the visited chunks in the LDS left below 40 KB (four
+    // workgroups per CU), or below 52 KB when the rest already exceeds it
+    k.ppc = a->page_size >= kChunk ? 1 : 4;
+    k.pages_off = (int)((n + 15) / 16 * 16);
+    const size_t budget = k.pages_off <= 40 * 1024 - 64 ? 40 * 1024 : 52 * 1024;
+    k.page_cap = (int)std::min<int64_t>(umax, k.pages_off < (int)budget ? (budget - k.pages_off) / (4 * k.ppc) : 0);
+    n = k.pages_off + (size_t)k.page_cap * 4 * k.ppc;
+    smem = (n + 15) / 16 * 16;
+    return std::min<int>(4, (int)((160 * 1024) / smem));
+  };
+  // The V pitch without conflicts, unless the launch needs more rounds with it
+  // than with the shorter one.  Ten heads, biased rows of their own selections,
+  // wide -> narrow, us: 5,000 rows of one request (790 tiles; 768 fit three to a
+  // CU) 148 -> 100; 16,000 rows 305 -> 272; four requests of 2,048 rows after
+  // 30,000 keys 181 -> 164.  The same workgroups per CU either way: 2,048 rows
+  // after 62,000 keys 182 -> 184, twelve slots 245 -> 247; one round: 4,000 rows
+  // 90.8 -> 91.5.
+  const size_t wide = a->D == 128 ? FwdLds<128>::tileBytes : FwdLds<64>::tileBytes;
+  const size_t narrow = a->D == 128 ? FwdLds<128, 2, true>::tileBytes : FwdLds<64, 2, true>::tileBytes;
+  int per_cu = layout(wide);
+  const bool fits = smem <= 156 * 1024;
+  if (!fits || (per_cu < 4 && nlogical > (int64_t)cus * per_cu)) {
+    const int with_narrow = layout(narrow);
+    k.narrow = !fits || with_narrow > per_cu;
+    per_cu = k.narrow ? with_narrow : layout(wide);
+  }
   if (smem > 156 * 1024) {
     set_error("paged fwd: %zu bytes of LDS needed (block table too wide)", smem);
     return SRSWA_UNSUPPORTED;
   }
   // every tile is split or none: which tiles are live is known on the device only
   k.nsplit = 1;
-  const int cus = device_cu_count();
-  const int per_cu = std::min<int>(4, (int)((160 * 1024) / smem));
   if (cus > 0 && per_cu > 0) k.nsplit = split_parts(nlogical, (int64_t)cus * per_cu, true);
   if (k.nsplit > 1) {
     k.ntail = k.nlogical;
@@ -1022,15 +1047,9 @@ extern "C" int srswa_gather_fwd_paged_ws(const srswa_paged_fwd_args* a, void* ws
   k.part = reinterpret_cast<float*>(ws);
   const bool fp8 = a->kv_fp8 != 0;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (fp8) {
-    if (a->dtype == SRSWA_BF16)
-      return a->D == 128 ? launch_fwd<bf16_t, 128, true, true>(k, smem, s)
-                         : launch_fwd<bf16_t, 64, true, true>(k, smem, s);
-    return a->D == 128 ? launch_fwd<__half, 128, true, true>(k, smem, s) : launch_fwd<__half, 64, true, true>(k, smem, s);
-  }
   if (a->dtype == SRSWA_BF16)
-    return a->D == 128 ? launch_fwd<bf16_t, 128, true>(k, smem, s) : launch_fwd<bf16_t, 64, true>(k, smem, s);
-  return a->D == 128 ? launch_fwd<__half, 128, true>(k, smem, s) : launch_fwd<__half, 64, true>(k, smem, s);
+    return fp8 ? launch_fwd_paged<bf16_t, true>(k, smem, s) : launch_fwd_paged<bf16_t, false>(k, smem, s);
+  return fp8 ? launch_fwd_paged<__half, true>(k, smem, s) : launch_fwd_paged<__half, false>(k, smem, s);
 }
 
 extern "C" int srswa_gather_fwd_paged(const srswa_paged_fwd_args* a, void* stream) {
