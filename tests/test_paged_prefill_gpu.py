@@ -206,3 +206,16 @@ def test_more_rounds_than_one_match_short_launches(dev, monkeypatch, D, K, page,
     second = _attend(c, [(0, 25 * 64, 24 * 64 - 5)])
     assert torch.isfinite(whole.float()).all()
     assert torch.equal(whole, torch.cat([first, second]))
+
+
+@pytest.mark.parametrize("H,rows", [(1, 1), (1, 700), (3, 64), (3, 321), (10, 65), (10, 1000)])
+def test_one_request_matches_itself_beside_another(dev, monkeypatch, H, rows):
+    """The tiles of one request are dealt to the XCDs in eighths, those of
+    several in turn (tile counts that are no multiple of eight, fewer than
+    eight, one): the same rows to the last bit.  (Without the split.)"""
+    from srswa import _lib
+    monkeypatch.setattr(_lib.lib(), "srswa_gather_fwd_paged_workspace", lambda a: 0)
+    c = _request_case(dev, rows, [rows, 1], [900, 70], H=H, HKV=H, D=128, page=64, K=5, dtype=torch.bfloat16)
+    alone, beside = _attend(c, [(0, 0, rows)]), _attend(c)
+    assert torch.isfinite(beside.float()).all() and alone.abs().amax(-1).min() > 0
+    assert torch.equal(alone, beside[:rows])
