@@ -104,10 +104,9 @@ def test_fwd_fp32_matches_oracle(dev, name):
 
 @pytest.mark.parametrize("name", ["self_bs64", "bias", "gqa_hi"])
 def test_tail_split_matches_whole_tiles(dev, name):
-    """The tail split (a last round of tiles filling at most a fifth of the GPU
-    runs as four workgroups per tile over quarters of their key chunks, then a
-    merge) against every tile whole and the oracle: these small launches are
-    one such round, so the split takes every tile."""
+    """The split (the tiles of a launch that leaves CUs idle run as several
+    workgroups over parts of their key chunks, then a merge) against every tile
+    whole and the oracle: these small launches run every tile as two."""
     import ctypes
     from srswa import _lib
     c = dict(CASES[name])
@@ -146,3 +145,59 @@ def test_tail_split_matches_whole_tiles(dev, name):
     cus = torch.cuda.get_device_properties(dev).multi_processor_count
     nws = _lib.lib().srswa_gather_fwd_workspace(ctypes.byref(a))
     assert (nws > 0) == (ntiles * 5 <= 4 * cus), (nws, ntiles, cus)
+
+
+BF, HF, F32 = torch.bfloat16, torch.float16, torch.float32
+
+
+@pytest.mark.parametrize("B,HQ,T,Sk,D,dtype,bias,tail,parts", [
+    (1, 4, 512, 760, 128, BF, False, 32, 8),      # 32 tiles: one part per CU
+    (2, 10, 320, 2500, 64, HF, True, 100, 8),     # long lists
+    (1, 10, 320, 960, 128, BF, True, 50, 4),
+    (1, 10, 250, 250, 128, BF, False, 40, 2),     # lists of one to four chunks
+    (1, 16, 1600, 1601, 128, HF, True, 400, 2),
+    (1, 10, 64, 64, 128, BF, False, 0, 1),        # one chunk: nothing to split
+    (1, 16, 2112, 2200, 128, BF, False, 0, 1),    # more tiles than half of the slots
+    (1, 16, 4150, 4150, 128, BF, True, 16, 4),    # 16 tiles past a full round, the others whole
+    (1, 4, 128, 128, 128, F32, False, 8, 2),
+    (1, 10, 250, 250, 128, F32, True, 40, 4),
+    (1, 10, 320, 320, 128, F32, True, 50, 8),
+])
+def test_split_launch_matches_whole_tiles(dev, B, HQ, T, Sk, D, dtype, bias, tail, parts):
+    """Each number of parts, the last round of several beside whole tiles, and
+    a launch too short or too full to split (256 CUs), against every tile whole.
+    Each probability is rounded to the 16-bit type (half a unit in the last
+    place, u: 2^-9 or 2^-12 of it) relative to its part's own reference maximum:
+    the two forms are at most 2 u sum(p |v|) <= 2 u max|v| apart before the
+    output's own rounding.  fp32 rounds none of them; its sums of up to 4,000
+    terms, in another order, differ by less than 1e-5 of max|v|."""
+    import ctypes
+    from srswa import _lib
+    g = torch.Generator(device=dev).manual_seed(T)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev).to(dtype)
+    q, k, v, S = rnd(B, T, HQ, D), rnd(B, Sk, HQ, D), rnd(B, Sk, HQ, D), 4
+    idx = torch.randint(-1, -(-Sk // 64), (B, 1, T, S), generator=g, device=dev).to(torch.int32)
+    args = dict(block_size=64, local_window=128, scale=D ** -0.5,
+                bias=torch.randn(B, T, S, generator=g, device=dev) if bias else None)
+    o_s, l_s = ops.gather_fwd(q, k, v, idx, **args)
+    o_w, l_w = ops.gather_fwd(q, k, v, idx, tail_split=False, **args)
+    a = _lib.FwdArgs()
+    a.B, a.T, a.Sk, a.HQ, a.HKV, a.HI, a.D, a.S = B, T, Sk, HQ, HQ, 1, D, S
+    a.q = a.k = a.v = a.out = q.data_ptr()
+    a.idx = idx.data_ptr()
+    a.bias = idx.data_ptr() if bias else None
+    a.block_size, a.local_window, a.scale, a.dtype = 64, 128, D ** -0.5, _lib.dtype_code(dtype)
+    assert _lib.lib().srswa_gather_fwd_workspace(ctypes.byref(a)) == tail * parts * (64 * D + 128) * 4
+    if parts == 1:
+        assert torch.equal(o_s, o_w) and torch.equal(l_s, l_w)
+        return
+    o_s, o_w, vmax = o_s.float(), o_w.float(), v.float().abs().max()
+    if dtype == F32:
+        bar, lse_bar = 1e-5 * vmax, 1e-5
+    else:
+        digits = 8 if dtype == BF else 11
+        ulp = torch.exp2(torch.floor(torch.log2(o_w.abs().clamp(min=1e-3))) - (digits - 1))
+        bar, lse_bar = 2.0 ** -digits * vmax + ulp, 1e-4
+    assert torch.isfinite(o_s).all() and ((o_s - o_w).abs() <= bar).all()
+    assert (l_s - l_w).abs().max().item() <= lse_bar
+    assert not torch.equal(l_s, l_w)              # the split did run

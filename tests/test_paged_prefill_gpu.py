@@ -219,3 +219,39 @@ def test_one_request_matches_itself_beside_another(dev, monkeypatch, H, rows):
     alone, beside = _attend(c, [(0, 0, rows)]), _attend(c)
     assert torch.isfinite(beside.float()).all() and alone.abs().amax(-1).min() > 0
     assert torch.equal(alone, beside[:rows])
+
+
+BF, HF = torch.bfloat16, torch.float16
+
+
+@pytest.mark.parametrize("H,HKV,D,page,K,dtype,kv,bias,q_lens,ctx,parts", [
+    (8, 2, 64, 16, 6, HF, None, False, [320, 1, 65], [700, 0, 300], 8),
+    (8, 8, 128, 32, 4, BF, None, False, [320, 1, 65], [700, 0, 300], 8),
+    (6, 3, 64, 64, 5, BF, torch.float8_e5m2, True, [130], [640], 8),
+    (16, 4, 64, 32, 5, HF, None, False, [400, 3], [300, 900], 4),
+    (16, 4, 128, 16, 5, HF, None, True, [640, 3], [100, 2000], 2),
+    (10, 10, 128, 64, 8, BF, None, True, [250], [0], 2),          # a table of four chunks
+    (10, 10, 128, 64, 8, BF, None, True, [60], [0], 1),           # of one: nothing to split
+])
+def test_split_forms_match_whole_tiles(dev, monkeypatch, H, HKV, D, page, K, dtype, kv, bias, q_lens, ctx, parts):
+    """The split over head dims, types, head groups, page sizes and the number of
+    parts (256 CUs), with and without bias, against every tile whole.  Bar as
+    in test_split_launch_matches_whole_tiles: 2 u max|v| and one unit in the
+    output's last place, u the 16-bit type's rounding of a probability."""
+    from srswa import _lib
+    real, asked = _lib.lib().srswa_gather_fwd_paged_workspace, []
+    c = _request_case(dev, sum(q_lens), q_lens, ctx, H=H, HKV=HKV, D=D, page=page, K=K, dtype=dtype, kv=kv, bias=bias)
+    monkeypatch.setattr(_lib.lib(), "srswa_gather_fwd_paged_workspace", lambda a: asked.append(real(a)) or asked[-1])
+    split = _attend(c)
+    monkeypatch.setattr(_lib.lib(), "srswa_gather_fwd_paged_workspace", lambda a: 0)
+    whole = _attend(c)
+    tiles = len(q_lens) * H * -(-max(q_lens) // 64)
+    assert asked == [0 if parts == 1 else tiles * parts * (64 * D + 128) * 4]
+    if parts == 1:
+        assert torch.equal(split, whole)
+        return
+    split, whole, vmax = split.float(), whole.float(), c["v"].float().abs().max()
+    digits = 8 if dtype == BF else 11
+    ulp = torch.exp2(torch.floor(torch.log2(whole.abs().clamp(min=1e-3))) - (digits - 1))
+    assert torch.isfinite(split).all() and ((split - whole).abs() <= 2.0 ** -digits * vmax + ulp).all()
+    assert not torch.equal(split, whole)          # the split did run

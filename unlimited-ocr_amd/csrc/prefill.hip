@@ -775,18 +775,39 @@ using namespace srswa;
 namespace srswa {
 namespace {
 
-// Parts per tile of a round of `tiles` tiles on a GPU that holds `slots`
-// workgroups.  A launch of one round (`alone`) takes as many of 8, 4 or 2 as
-// the slots hold: a tile's chunks are a chain of load latencies, and idle CUs
-// run the parts at once.  One request behind 30,000 keys, ten heads, biased
-// rows of their own selections (17 to 21 chunks a tile), whole -> split: 40
-// tiles 70 -> 28 us (8 parts), 120 tiles 71 -> 41 (4), 190 tiles 71 -> 46 (4),
-// 250 tiles 71 -> 58 (2), 380 tiles 86 -> 67 (2).  The last round of several
-// only up to a fifth of the slots, in 4 parts: see below.
-int split_parts(int64_t tiles, int64_t slots, bool alone) {
-  if (!alone) return tiles * 5 <= slots ? 4 : 1;
-  return tiles * 8 <= slots ? 8 : tiles * 4 <= slots ? 4 : tiles * 2 <= slots ? 2 : 1;
+// Parts per tile of a launch of one round, `tiles` tiles on a GPU of `cus` CUs
+// that holds `slots` workgroups: as many of 8, 4 or 2 as the slots hold and the
+// chunk lists pay for.  A tile's chunks are a chain of load latencies, and idle
+// CUs run the parts at once; each part repeats the set-up and writes a record,
+// and a merge is launched.  `chunks2` is twice the mean length that the lists
+// can have.  One request behind 30,000 keys, ten heads, biased rows of their own
+// selections (17 to 21 chunks a tile), whole -> split: 40 tiles 70 -> 28 us (8
+// parts), 120 tiles 71 -> 41 (4), 190 tiles 71 -> 46 (4), 250 tiles 71 -> 58 (2),
+// 380 tiles 86 -> 67 (2).  Where the lines lie, in us for 1 / 2 / 4 / 8 parts:
+//   1 chunk, 10 tiles: 9.0 / 11.1 / 11.6 / 12.9
+//   1 to 2, 32 tiles: 10.6 / 11.9 / 13.1 / 15.8
+//   1 to 4, 40 tiles: 13.7 / 13.6 / 13.7 / 18.5, paged 16.2 / 14.6 / 13.6 / 17.1
+//   5, 10 tiles: 15.3 / 14.3 / 13.3 / 13.0
+//   5 to 8, 64 tiles: 19.9 / 18.1 / 17.4 / 22.0
+//   10 to 12, 32 tiles (8 parts: one per CU): 28.5 / 21.4 / 17.8 / 18.7, paged 35.5 / 24.5 / 18.9 / 18.4
+//   11 to 15, 50 tiles: 34.4 / 25.3 / 22.1 / 23.7, paged 43.0 / 29.5 / 22.7 / 24.1
+//   17, 50 tiles: 41.6 / 29.5 / 24.4 / 27.1
+//   17 to 21, 50 tiles: 56.7 / 39.2 / 29.4 / 27.6, paged 69.5 / 45.9 / 32.3 / 29.5
+// fp32, where a chunk takes about four times as long:
+//   1 to 2, 32 tiles: 25.5 / 19.7 / 21.0 / 23.4
+//   1 to 4, 40 tiles: 42.8 / 28.5 / 21.8 / 26.3
+//   1 to 5, 50 tiles: 51.7 / 37.4 / 30.8 / 27.5
+int split_parts(int64_t tiles, int64_t slots, int64_t cus, int chunks2, bool f32, bool paged) {
+  const int for8 = f32 ? 6 : tiles * 8 <= cus ? 10 : paged ? 24 : 32;
+  if (tiles * 8 <= slots && chunks2 >= for8) return 8;
+  if (tiles * 4 <= slots && chunks2 >= (f32 ? 4 : 10)) return 4;
+  return tiles * 2 <= slots && chunks2 >= (f32 ? 3 : 4) ? 2 : 1;
 }
+
+// Twice the mean number of chunks that the tiles of a request can visit: the
+// last tile reaches all nchunk of its keys, each one before it at least a chunk
+// less, and none more than umax.
+int mean_chunks2(int nchunk, int ntiles, int umax) { return std::min(2 * umax, 2 * nchunk - (ntiles - 1)); }
 
 // The forward's launch plan (no device work).  Returns SRSWA_OK with k, smem
 // and the split's workspace bytes filled in.
@@ -825,9 +846,10 @@ int plan_fwd(const srswa_fwd_args* a, FwdK& k, size_t& smem, size_t& ws_bytes) {
     set_error("fwd: %zu bytes of LDS needed (key length too large)", smem);
     return SRSWA_UNSUPPORTED;
   }
-  // Split of the last round.  The GPU holds `slots` workgroups at once (four
-  // per CU at two waves per SIMD, fewer when LDS runs out).  When the last
-  // round of several fills at most a fifth of them, its tiles run as four
+  // Split of a single round (split_parts) or of the last of several.  The GPU
+  // holds `slots` workgroups at once (four per CU at two waves per SIMD, fewer
+  // when LDS runs out).  When the last of several rounds fills at most a fifth
+  // of them, its tiles run as four
   // workgroups each over quarters of their chunk plans, so that round takes
   // about a quarter of a tile's time.  A fuller last round is left whole: each
   // part pays the tile's set-up and first-load latency again, and its fp32
@@ -843,7 +865,8 @@ int plan_fwd(const srswa_fwd_args* a, FwdK& k, size_t& smem, size_t& ws_bytes) {
     const int64_t slots = (int64_t)cus * per_cu;
     const int64_t rounds = (nlogical + slots - 1) / slots;
     const int64_t tail = nlogical - (rounds - 1) * slots;
-    k.nsplit = split_parts(tail, slots, rounds == 1);
+    k.nsplit = rounds == 1 ? split_parts(tail, slots, cus, mean_chunks2(nchunk, k.ntiles, umax), f32, false)
+                           : tail * 5 <= slots ? 4 : 1;
     if (k.nsplit > 1) {
       k.ntail = (int)tail;
       ws_bytes = (size_t)tail * k.nsplit * (64 * a->D + 128) * sizeof(float);
@@ -1034,9 +1057,13 @@ int plan_fwd_paged(const srswa_paged_fwd_args* a, FwdK& k, size_t& smem, size_t&
     set_error("paged fwd: %zu bytes of LDS needed (block table too wide)", smem);
     return SRSWA_UNSUPPORTED;
   }
-  // every tile is split or none: which tiles are live is known on the device only
+  // Every tile is split or none: which tiles are live is known on the device
+  // only.  So is the requests' length: the table's width bounds the chunks, and
+  // tiles past the end of the shorter requests count (a batch of one long and
+  // many short requests that would leave CUs idle may run whole).
   k.nsplit = 1;
-  if (cus > 0 && per_cu > 0) k.nsplit = split_parts(nlogical, (int64_t)cus * per_cu, true);
+  if (cus > 0 && per_cu > 0)
+    k.nsplit = split_parts(nlogical, (int64_t)cus * per_cu, cus, mean_chunks2(nchunk, k.ntiles, umax), false, true);
   if (k.nsplit > 1) {
     k.ntail = k.nlogical;
     ws_bytes = (size_t)nlogical * k.nsplit * (64 * a->D + 128) * sizeof(float);
