@@ -79,8 +79,8 @@ __host__ __device__ __forceinline__ bool eighths_deal(const FwdK& p) { return p.
 // a 4-float pad keeps the two lane halves' rows, 4 apart, on different banks)
 // NARROW gives up the V pitch without conflicts for 1 KB: the paged form with
 // slot biases and page ids can then stay within 40 KB, four workgroups per CU
-// instead of three.  The plan takes it only where that lets the launch run in
-// fewer rounds (plan_fwd_paged).
+// instead of three.  The plan takes it only where that saves a round or lets
+// the tiles run in more parts (plan_fwd_paged).
 template <int D, int ES = 2, bool NARROW = false> struct FwdLds {
   static constexpr int KP = D + 8;                  // K row pitch (elements): conflict-free row reads
   static constexpr int VP = ES == 4 ? D + 4 : NARROW ? D + 8 : D + 16;   // V row pitch: conflict-free V^T reads at + 16
@@ -1038,32 +1038,36 @@ int plan_fwd_paged(const srswa_paged_fwd_args* a, FwdK& k, size_t& smem, size_t&
     return std::min<int>(4, (int)((160 * 1024) / smem));
   };
   // The V pitch without conflicts, unless the launch needs more rounds with it
-  // than with the shorter one.  Ten heads, biased rows of their own selections,
-  // wide -> narrow, us: 5,000 rows of one request (790 tiles; 768 fit three to a
-  // CU) 148 -> 100; 16,000 rows 305 -> 272; four requests of 2,048 rows after
-  // 30,000 keys 181 -> 164.  The same workgroups per CU either way: 2,048 rows
-  // after 62,000 keys 182 -> 184, twelve slots 245 -> 247; one round: 4,000 rows
-  // 90.8 -> 91.5.
+  // than with the shorter one, or runs in fewer parts.  Ten heads, biased rows of
+  // their own selections, wide -> narrow, us: 5,000 rows of one request (790
+  // tiles; 768 fit three to a CU) 148 -> 100; 16,000 rows 305 -> 272; four requests
+  // of 2,048 rows after 30,000 keys 181 -> 164; one of 2,560 rows (whole -> two
+  // parts) 85 -> 69, of 1,472 (two -> four) 57 -> 50.  The same workgroups per CU
+  // either way: 2,048 rows after 62,000 keys 182 -> 184, twelve slots 245 -> 247;
+  // one round, whole either way: 4,000 rows 90.8 -> 91.5.
   const size_t wide = a->D == 128 ? FwdLds<128>::tileBytes : FwdLds<64>::tileBytes;
   const size_t narrow = a->D == 128 ? FwdLds<128, 2, true>::tileBytes : FwdLds<64, 2, true>::tileBytes;
+  // Every tile is split or none: which tiles are live is known on the device
+  // only.  So is the requests' length: the table's width bounds the chunks, and
+  // tiles past the end of the shorter requests count (a batch of one long and
+  // many short requests that would leave CUs idle may run whole).
+  auto parts = [&](int per_cu) {
+    if (cus <= 0 || per_cu <= 0) return 1;
+    return split_parts(nlogical, (int64_t)cus * per_cu, cus, mean_chunks2(nchunk, k.ntiles, umax), false, true);
+  };
   int per_cu = layout(wide);
   const bool fits = smem <= 156 * 1024;
-  if (!fits || (per_cu < 4 && nlogical > (int64_t)cus * per_cu)) {
+  if (!fits || per_cu < 4) {
     const int with_narrow = layout(narrow);
-    k.narrow = !fits || with_narrow > per_cu;
+    k.narrow = !fits || (with_narrow > per_cu &&
+                         (nlogical > (int64_t)cus * per_cu || parts(with_narrow) > parts(per_cu)));
     per_cu = k.narrow ? with_narrow : layout(wide);
   }
   if (smem > 156 * 1024) {
     set_error("paged fwd: %zu bytes of LDS needed (block table too wide)", smem);
     return SRSWA_UNSUPPORTED;
   }
-  // Every tile is split or none: which tiles are live is known on the device
-  // only.  So is the requests' length: the table's width bounds the chunks, and
-  // tiles past the end of the shorter requests count (a batch of one long and
-  // many short requests that would leave CUs idle may run whole).
-  k.nsplit = 1;
-  if (cus > 0 && per_cu > 0)
-    k.nsplit = split_parts(nlogical, (int64_t)cus * per_cu, cus, mean_chunks2(nchunk, k.ntiles, umax), false, true);
+  k.nsplit = parts(per_cu);
   if (k.nsplit > 1) {
     k.ntail = k.nlogical;
     ws_bytes = (size_t)nlogical * k.nsplit * (64 * a->D + 128) * sizeof(float);
