@@ -266,7 +266,7 @@ def test_block_max_scores_fwd_bwd(dev, name):
                                   "integer_ties_clamped_bs64"])
 def test_block_max_backward_few_gradients(dev, name, share):
     """Most upstream gradients zero, as behind the router: both forms of dq (a
-    wave takes the first when its rows weigh at most half of a group's blocks;
+    wave takes the first when its rows weigh at most 7/16 of a group's blocks;
     ``share`` lies on either side) and short and long lists of dk, ties among them."""
     from srswa import train_scores as TS
     q, k, pos, nblk, bs, lw = _bm_case(name)

@@ -51,8 +51,8 @@
 // bm_fwd (128 rows per workgroup, 64-key chunks through LDS, S^T = K Q^T on
 // v_mfma_f32_32x32x2_f32 as the inference block-max kernel, then per block the
 // clamped max, its tie and in-range masks), bm_bwd_dq (4 rows per wave, 16
-// waves per 64-row tile, the arg-max key rows of two blocks gathered
-// together) and bm_bwd_dk (a workgroup per block, four keys per wave, 16 lanes
+// waves per 64-row tile, the arg-max key rows of a block or of a row's few
+// blocks gathered together) and bm_bwd_dk (a workgroup per block, four keys per wave, 16 lanes
 // each, scanning the block's codes in row order).  No atomics: every result is deterministic.
 #include <algorithm>
 #include <climits>
@@ -898,19 +898,24 @@ __device__ __forceinline__ int bm_last_remote(int p, int LW, int BS) { return p 
 // blocks the codes and weights g / n are staged in LDS (and the weights stored
 // block-major for bm_bwd_dk).  Behind the router a row's gradient reaches the
 // few blocks of its entmax support and every other weight is exactly zero: a
-// wave whose rows weigh at most half of the group's blocks takes only those,
+// wave whose rows weigh at most 7/16 of the group's blocks takes only those,
 // row by row, the key rows of kBmBatch of them loaded together (lanes over the
 // head dims); otherwise every block, the key rows of kBmBpi blocks and all
-// four rows together.  Both add in block order.  B = 2, S = 16384, 256 blocks,
-// the router's gradients: 157 us walking every block, 64 now; a gradient in
-// every block 276 and 291 us (361 when it took the first form too).
+// four rows together.  Both add in block order.  The gathers are load
+// latencies: at most 64 registers let a CU hold two workgroups.  B = 2, S =
+// 16384, 256 blocks, us by the share of (row, block) gradients, walking every
+// block alone (one workgroup per CU) / now: the router's 160 / 36, 0.1 166 / 67,
+// 0.3 188 / 132, 0.45 203 / 207, 0.55 212 / 218, 0.7 225 / 236, 1 268 / 267.
+// The few-blocks form meets the other near 0.45 (206; half as the line and one
+// workgroup per CU: 238 at 0.45, 250 at 0.55).  Batches of 3, 4 and 8: 38, 40
+// and 46 at the router's; two blocks per step in the other form: 270 at 1.
 constexpr int kBmRpw = 4;                               // rows per wave
 constexpr int kBmDqWaves = kTsRows / kBmRpw;
-constexpr int kBmBatch = 8;                             // few blocks: key rows loaded together
-constexpr int kBmBpi = 2;                               // every block: blocks gathered together (divides kTsGroup)
+constexpr int kBmBatch = 2;                             // few blocks: key rows loaded together
+constexpr int kBmBpi = 1;                               // every block: blocks gathered together (divides kTsGroup)
 
 template <int D, int BS>
-__global__ __launch_bounds__(kBmDqWaves * kWave) void bm_bwd_dq_kernel(BmBK p) {
+__global__ __launch_bounds__(kBmDqWaves * kWave, 8) void bm_bwd_dq_kernel(BmBK p) {
   constexpr int EPL = D / kWave;
   __shared__ int s_code[kTsGroup * kTsPad];     // [block][row]
   __shared__ float s_w[kTsGroup * kTsPad];      // [block][row]
@@ -995,7 +1000,7 @@ __global__ __launch_bounds__(kBmDqWaves * kWave) void bm_bwd_dq_kernel(BmBK p) {
       live[r] = __ballot(w_l[r] != 0.f);
       total += __popcll(live[r]);
     }
-    if (total * 2 <= cn * kBmRpw) {
+    if (total * 16 <= cn * kBmRpw * 7) {
 #pragma unroll
       for (int r = 0; r < kBmRpw; ++r) {
         while (live[r]) {
