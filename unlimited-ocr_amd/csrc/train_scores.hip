@@ -1093,15 +1093,19 @@ __device__ __forceinline__ void wave_sync_lds() {
 // at a time (the next rows loaded while these are taken).  Every wave scans
 // them 64 rows at a time in row order and lists the rows whose gradient
 // reaches each of its keys; when a list may not hold 64 more, every lane group
-// adds up its key's list, kDkBatch query rows loaded together.  B = 2, S =
-// 16384, 256 blocks, a gradient in every block: 255 us, and 329 with each wave
-// reading the column for itself and adding the rows of every 64 as it met
-// them, one load latency after the other; the router's gradients 109 and 105.
+// adds up its key's list, kDkBatch query rows loaded together.  Most rows reach
+// the first blocks, whose lists are the longest: every sequence's first blocks
+// are dispatched first.  At most 64 registers: two workgroups per CU.
+// B = 2, S = 16384, 256 blocks, a gradient in every block / the router's
+// gradients: 227 / 93 us; one sequence's blocks after the other's, one workgroup
+// per CU and batches of four 246 / 117; each wave reading the column for itself
+// and adding the rows of every 64 as it met them, one load latency after the
+// other, 326 / 105.
 constexpr int kDkList = 96;     // list entries per key
-constexpr int kDkBatch = 4;
+constexpr int kDkBatch = 3;
 
 template <int D, int BS>
-__global__ __launch_bounds__(16 * BS) void bm_bwd_dk_kernel(BmBK p) {
+__global__ __launch_bounds__(16 * BS, 8) void bm_bwd_dk_kernel(BmBK p) {
   constexpr int DPL = D / 16;                    // head dims per lane
   constexpr int NT = 16 * BS;                    // threads, and rows per batch
   __shared__ int s_code[2][NT];
@@ -1109,9 +1113,8 @@ __global__ __launch_bounds__(16 * BS) void bm_bwd_dk_kernel(BmBK p) {
   __shared__ __align__(16) int2 s_list[BS][kDkList];   // per key: (row, weight bits), rows ascending
   const srswa_bm_score_bwd_args& a = p.a;
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
-  const int nblk_keys = min(a.nblk, ceil_div(a.S, BS));
-  const int blk = (int)blockIdx.x % nblk_keys;
-  const int b = (int)blockIdx.x / nblk_keys;
+  const int blk = (int)blockIdx.x / a.B;
+  const int b = (int)blockIdx.x % a.B;
   const int kgrp = lane / 16, dl = lane % 16;
   const int off0 = 4 * wave;                      // first key offset of the wave's four
   const int my_key = off0 + kgrp;
