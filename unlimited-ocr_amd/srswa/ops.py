@@ -622,8 +622,10 @@ def _seg_from_positions(position_ids, T, Sk, device):
         return None
     qi = torch.arange(Sk - T, Sk, device=device, dtype=torch.int64)
     pos = position_ids.to(device=device, dtype=torch.int64)
-    out = torch.empty(torch.broadcast_shapes((1, T), pos.shape), dtype=torch.int32, device=device)
-    return torch.sub(qi[None], pos, out=out)                             # narrowed as it is stored
+    if pos.dim() < 2:
+        pos = pos.expand(1, T)
+    out = torch.empty((*pos.shape[:-1], T), dtype=torch.int32, device=device)
+    return torch.sub(qi, pos, out=out)                                   # narrowed as it is stored
 
 
 def gather_fwd(q, k, v, block_indices, *, block_size, local_window, scale, seg=None, bias=None,
