@@ -106,7 +106,7 @@ def test_fwd_fp32_matches_oracle(dev, name):
 def test_tail_split_matches_whole_tiles(dev, name):
     """The split (the tiles of a launch that leaves CUs idle run as several
     workgroups over parts of their key chunks, then a merge) against every tile
-    whole and the oracle: these small launches run every tile as two."""
+    whole and the oracle: these small launches run every tile as four."""
     import ctypes
     from srswa import _lib
     c = dict(CASES[name])
@@ -154,7 +154,8 @@ BF, HF, F32 = torch.bfloat16, torch.float16, torch.float32
     (1, 4, 512, 760, 128, BF, False, 32, 8),      # 32 tiles: one part per CU
     (2, 10, 320, 2500, 64, HF, True, 100, 8),     # long lists
     (1, 10, 320, 960, 128, BF, True, 50, 4),
-    (1, 10, 250, 250, 128, BF, False, 40, 2),     # lists of one to four chunks
+    (1, 10, 250, 250, 128, BF, False, 40, 4),     # lists of one to four chunks
+    (1, 16, 250, 250, 128, BF, False, 64, 2),
     (1, 16, 1600, 1601, 128, HF, True, 400, 2),
     (1, 10, 64, 64, 128, BF, False, 0, 1),        # one chunk: nothing to split
     (1, 16, 2112, 2200, 128, BF, False, 0, 1),    # more tiles than half of the slots

@@ -208,11 +208,12 @@ def test_more_rounds_than_one_match_short_launches(dev, monkeypatch, D, K, page,
     assert torch.equal(whole, torch.cat([first, second]))
 
 
-@pytest.mark.parametrize("H,rows", [(1, 1), (1, 700), (3, 64), (3, 321), (10, 65), (10, 1000)])
+@pytest.mark.parametrize("H,rows", [(1, 1), (1, 700), (3, 64), (3, 321), (10, 65), (10, 1000), (4, 700), (8, 321)])
 def test_one_request_matches_itself_beside_another(dev, monkeypatch, H, rows):
     """The tiles of one request are dealt to the XCDs in eighths, those of
     several in turn (tile counts that are no multiple of eight, fewer than
-    eight, one): the same rows to the last bit.  (Without the split.)"""
+    eight, one; requests times heads 8 and 16, where a head's tiles stay on one
+    XCD): the same rows to the last bit.  (Without the split.)"""
     from srswa import _lib
     monkeypatch.setattr(_lib.lib(), "srswa_gather_fwd_paged_workspace", lambda a: 0)
     c = _request_case(dev, rows, [rows, 1], [900, 70], H=H, HKV=H, D=128, page=64, K=5, dtype=torch.bfloat16)
@@ -230,7 +231,8 @@ BF, HF = torch.bfloat16, torch.float16
     (6, 3, 64, 64, 5, BF, torch.float8_e5m2, True, [130], [640], 8),
     (16, 4, 64, 32, 5, HF, None, False, [400, 3], [300, 900], 4),
     (16, 4, 128, 16, 5, HF, None, True, [640, 3], [100, 2000], 2),
-    (10, 10, 128, 64, 8, BF, None, True, [250], [0], 2),          # a table of four chunks
+    (10, 10, 128, 64, 8, BF, None, True, [250], [0], 4),          # a table of four chunks
+    (16, 16, 128, 64, 8, BF, None, True, [250], [0], 2),
     (10, 10, 128, 64, 8, BF, None, True, [60], [0], 1),           # of one: nothing to split
 ])
 def test_split_forms_match_whole_tiles(dev, monkeypatch, H, HKV, D, page, K, dtype, kv, bias, q_lens, ctx, parts):

@@ -786,7 +786,10 @@ namespace {
 // 380 tiles 86 -> 67 (2).  Where the lines lie, in us for 1 / 2 / 4 / 8 parts:
 //   1 chunk, 10 tiles: 9.0 / 11.1 / 11.6 / 12.9
 //   1 to 2, 32 tiles: 10.6 / 11.9 / 13.1 / 15.8
+//   1 to 3, 30 tiles: 12.0 / 13.2 / 12.9 / 15.5
 //   1 to 4, 40 tiles: 13.7 / 13.6 / 13.7 / 18.5, paged 16.2 / 14.6 / 13.6 / 17.1
+//   1 to 4, 64 tiles: 13.5 / 14.6 / 15.6 / 21.7, paged 16.1 / 15.2 / 15.3 / 19.5
+//   1 to 8, 80 tiles: 19.8 / 18.6 / 19.1 / 24.6, paged 24.4 / 20.1 / 20.8 / 22.1
 //   5, 10 tiles: 15.3 / 14.3 / 13.3 / 13.0
 //   5 to 8, 64 tiles: 19.9 / 18.1 / 17.4 / 22.0
 //   10 to 12, 32 tiles (8 parts: one per CU): 28.5 / 21.4 / 17.8 / 18.7, paged 35.5 / 24.5 / 18.9 / 18.4
@@ -800,7 +803,8 @@ namespace {
 int split_parts(int64_t tiles, int64_t slots, int64_t cus, int chunks2, bool f32, bool paged) {
   const int for8 = f32 ? 6 : tiles * 8 <= cus ? 10 : paged ? 24 : 32;
   if (tiles * 8 <= slots && chunks2 >= for8) return 8;
-  if (tiles * 4 <= slots && chunks2 >= (f32 ? 4 : 10)) return 4;
+  const int for4 = f32 || tiles * 5 <= cus ? 4 : 10;
+  if (tiles * 4 <= slots && chunks2 >= for4) return 4;
   return tiles * 2 <= slots && chunks2 >= (f32 ? 3 : 4) ? 2 : 1;
 }
 
