@@ -43,7 +43,7 @@ class _Launch:
         self.fn, self.args, self.keep, self.extra = fn, args, keep, extra
         self.stream, self.what = stream, what
         self._ref = ctypes.byref(args)
-        self._extra = tuple(_lib.ptr(x) if isinstance(x, torch.Tensor) else x for x in extra)
+        self._extra = [x.data_ptr() if isinstance(x, torch.Tensor) else x for x in extra]
 
     def __call__(self):
         _lib.check(self.fn(self._ref, *self._extra, self.stream), self.what)
@@ -69,10 +69,10 @@ def prepare_gather_decode(q, k_cache, v_cache, block_indices, q_pos, *, block_si
             q_pos = q_pos.unsqueeze(1)
     B, Lq, HQ, D = q.shape
     Bk, L, HKV, Dk = k_cache.shape
-    if Bk != B or Dk != D or tuple(v_cache.shape) != tuple(k_cache.shape):
+    if Bk != B or Dk != D or v_cache.shape != k_cache.shape:
         raise ValueError(f"cache shape {tuple(k_cache.shape)} / {tuple(v_cache.shape)} vs q {tuple(q.shape)}")
     HI, S = block_indices.shape[1], block_indices.shape[-1]
-    if tuple(block_indices.shape) != (B, HI, Lq, S):
+    if block_indices.shape != (B, HI, Lq, S):
         raise ValueError(f"block_indices shape {tuple(block_indices.shape)} != {(B, HI, Lq, S)}")
     if q.dtype != k_cache.dtype or q.dtype != v_cache.dtype:
         raise ValueError("q, k_cache, v_cache must share a dtype")
@@ -85,7 +85,7 @@ def prepare_gather_decode(q, k_cache, v_cache, block_indices, q_pos, *, block_si
     if valid is not None:
         valid = _as(valid, torch.bool, idx.shape).view(torch.uint8)
     pos = _i32(q_pos).contiguous()
-    if tuple(pos.shape) != (B, Lq):
+    if pos.shape != (B, Lq):
         raise ValueError(f"q_pos shape {tuple(pos.shape)} != {(B, Lq)}")
     kvl = None if kv_len is None else _i32(kv_len).contiguous()
     odt = out_dtype or q.dtype
@@ -195,7 +195,7 @@ def prepare_index_meanpool_topk(q, k, q_pos, *, block_size, local_blocks, topk, 
     nblk = int(nblk) if nblk is not None else -(-L // int(block_size))
     qf = q.to(torch.float32)
     pos = _i32(q_pos).contiguous()
-    if tuple(pos.shape) != (B, Lq):
+    if pos.shape != (B, Lq):
         raise ValueError(f"q_pos shape {tuple(pos.shape)} != {(B, Lq)}")
     kvl = None if kv_len is None else _i32(kv_len).contiguous()
     hc = None if head_cls is None else head_cls.to(torch.float32).contiguous()
@@ -306,7 +306,7 @@ def prepare_gather_decode_paged(q, k_cache, v_cache, topk_idx, blk_bias, block_t
     R = seq_lens.shape[0]
     if total_q != R * dql:
         raise ValueError(f"total_q {total_q} != {R} requests x {dql} queries")
-    if Dk != D or tuple(v_cache.shape) != tuple(k_cache.shape):
+    if Dk != D or v_cache.shape != k_cache.shape:
         raise ValueError(f"cache shape {tuple(k_cache.shape)} / {tuple(v_cache.shape)} vs q {tuple(q.shape)}")
     if topk_idx.dim() != 3 or topk_idx.shape[0] != HKV or topk_idx.shape[1] != total_q:
         raise ValueError(f"topk_idx shape {tuple(topk_idx.shape)} != ({HKV}, {total_q}, K)")
@@ -319,7 +319,7 @@ def prepare_gather_decode_paged(q, k_cache, v_cache, topk_idx, blk_bias, block_t
     ti = _i32(topk_idx)
     bias = None
     if blk_bias is not None:
-        if tuple(blk_bias.shape) != tuple(topk_idx.shape):
+        if blk_bias.shape != topk_idx.shape:
             raise ValueError(f"blk_bias shape {tuple(blk_bias.shape)} != topk_idx {tuple(topk_idx.shape)}")
         bias = blk_bias.to(torch.float32)
         if bias.stride() != ti.stride():
@@ -375,7 +375,7 @@ def gather_fwd_paged(q, k_cache, v_cache, topk_idx, blk_bias, block_table, cu_se
     _require_cuda(q, k_cache, v_cache, topk_idx, blk_bias, block_table, cu_seqlens_q, seq_lens, prefix_lens, out)
     total_q, HQ, D = q.shape
     npages, page, HKV, Dk = k_cache.shape
-    if Dk != D or tuple(v_cache.shape) != tuple(k_cache.shape):
+    if Dk != D or v_cache.shape != k_cache.shape:
         raise ValueError(f"cache shape {tuple(k_cache.shape)} / {tuple(v_cache.shape)} vs q {tuple(q.shape)}")
     if topk_idx.dim() != 3 or topk_idx.shape[0] != HKV or topk_idx.shape[1] != total_q:
         raise ValueError(f"topk_idx shape {tuple(topk_idx.shape)} != ({HKV}, {total_q}, K)")
@@ -388,7 +388,7 @@ def gather_fwd_paged(q, k_cache, v_cache, topk_idx, blk_bias, block_table, cu_se
         ti = ti.contiguous()
     bias = None
     if blk_bias is not None:
-        if tuple(blk_bias.shape) != tuple(topk_idx.shape):
+        if blk_bias.shape != topk_idx.shape:
             raise ValueError(f"blk_bias shape {tuple(blk_bias.shape)} != topk_idx {tuple(topk_idx.shape)}")
         bias = blk_bias.to(torch.float32)
         if bias.stride(-1) != 1:
@@ -640,7 +640,7 @@ def gather_fwd(q, k, v, block_indices, *, block_size, local_window, scale, seg=N
     _require_cuda(q, k, v, block_indices, seg, bias)
     B, T, HQ, D = q.shape
     Bk, Sk, HKV, Dk = k.shape
-    if Bk != B or Dk != D or tuple(v.shape) != tuple(k.shape):
+    if Bk != B or Dk != D or v.shape != k.shape:
         raise ValueError(f"k/v shape {tuple(k.shape)} incompatible with q {tuple(q.shape)}")
     if q.dtype != k.dtype or k.dtype != v.dtype:
         raise ValueError("q, k, v must share a dtype")
@@ -648,7 +648,7 @@ def gather_fwd(q, k, v, block_indices, *, block_size, local_window, scale, seg=N
         if t.stride(-1) != 1:
             raise UnsupportedShape("head dim must be contiguous")
     HI, S = block_indices.shape[1], block_indices.shape[-1]
-    if tuple(block_indices.shape) != (B, HI, T, S):
+    if block_indices.shape != (B, HI, T, S):
         raise ValueError(f"block_indices shape {tuple(block_indices.shape)} != {(B, HI, T, S)}")
     idx = _i32(block_indices).contiguous()
     if bias is not None:
