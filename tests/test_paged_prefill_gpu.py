@@ -234,6 +234,10 @@ BF, HF = torch.bfloat16, torch.float16
     (10, 10, 128, 64, 8, BF, None, True, [250], [0], 4),          # a table of four chunks
     (16, 16, 128, 64, 8, BF, None, True, [250], [0], 2),
     (10, 10, 128, 64, 8, BF, None, True, [60], [0], 1),           # of one: nothing to split
+    (10, 10, 128, 64, 8, BF, None, True, [168, 12], [64, 30], 4),
+    (10, 10, 128, 64, 8, BF, None, True, [250, 60, 100], [64, 0, 64], 2),
+    (10, 10, 128, 64, 8, BF, None, True, [120, 20, 12, 60, 90, 30, 15, 100], [150] * 8, 1),
+    (10, 10, 128, 64, 8, BF, None, True, [64, 1, 20, 33] * 3, [64] * 12, 1),
 ])
 def test_split_forms_match_whole_tiles(dev, monkeypatch, H, HKV, D, page, K, dtype, kv, bias, q_lens, ctx, parts):
     """The split over head dims, types, head groups, page sizes and the number of

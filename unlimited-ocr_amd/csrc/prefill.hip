@@ -790,6 +790,16 @@ namespace {
 //   1 to 4, 40 tiles: 13.7 / 13.6 / 13.7 / 18.5, paged 16.2 / 14.6 / 13.6 / 17.1
 //   1 to 4, 64 tiles: 13.5 / 14.6 / 15.6 / 21.7, paged 16.1 / 15.2 / 15.3 / 19.5
 //   1 to 8, 80 tiles: 19.8 / 18.6 / 19.1 / 24.6, paged 24.4 / 20.1 / 20.8 / 22.1
+// and several short requests in pages (tiles past a request's rows counted), each
+// behind 64 keys:
+//   two of 12 to 168 rows, 60 tiles: 16.3 / 15.2 / 12.9 / 16.0
+//   twelve of 1 to 64, 96 tiles: 12.9 / 13.9 / 15.8 / 21.0; 120 tiles: 12.6 / 14.2 / 16.7 / 23.4
+//   three of 60 to 250, 96 tiles: 23.3 / 20.3 / 18.6 / 22.0; 120 tiles: 20.1 / 18.4 / 20.6 / 23.7
+//   five of 12 to 168, 120 tiles: 19.0 / 17.2 / 17.1 / 21.0; 150 tiles: 16.5 / 18.3 / 19.6
+//   eight of 12 to 120, 128 tiles: 15.8 / 16.5 / 18.5 / 23.4; 160 tiles: 14.8 / 18.7 / 19.9
+//   the same behind 150 keys, 128 tiles: 19.4 / 18.1 / 19.2 / 23.4; 160 tiles: 16.9 / 19.2 / 20.4
+//   the same behind 250 keys, 128 tiles: 26.5 / 22.0 / 22.9 / 24.9; 160 tiles: 22.8 / 22.5 / 22.6
+// longer again:
 //   5, 10 tiles: 15.3 / 14.3 / 13.3 / 13.0
 //   5 to 8, 64 tiles: 19.9 / 18.1 / 17.4 / 22.0
 //   10 to 12, 32 tiles (8 parts: one per CU): 28.5 / 21.4 / 17.8 / 18.7, paged 35.5 / 24.5 / 18.9 / 18.4
@@ -803,9 +813,10 @@ namespace {
 int split_parts(int64_t tiles, int64_t slots, int64_t cus, int chunks2, bool f32, bool paged) {
   const int for8 = f32 ? 6 : tiles * 8 <= cus ? 10 : paged ? 24 : 32;
   if (tiles * 8 <= slots && chunks2 >= for8) return 8;
-  const int for4 = f32 || tiles * 5 <= cus ? 4 : 10;
+  const int for4 = f32 || tiles * 5 <= cus || (paged && tiles * 4 < cus) ? 4 : 10;
   if (tiles * 4 <= slots && chunks2 >= for4) return 4;
-  return tiles * 2 <= slots && chunks2 >= (f32 ? 3 : 4) ? 2 : 1;
+  const int for2 = f32 ? 3 : !paged || tiles * 4 <= cus ? 4 : tiles * 2 <= cus ? 6 : 10;
+  return tiles * 2 <= slots && chunks2 >= for2 ? 2 : 1;
 }
 
 // Twice the mean number of chunks that the tiles of a request can visit: the
