@@ -170,10 +170,10 @@ typedef struct {
 int srswa_gather_fwd(const srswa_fwd_args* a, void* stream);
 
 /* srswa_gather_fwd with a workspace for the split: when the launch's 64-row
- * tiles fill at most half of the GPU, or the last of several rounds of them at
- * most a fifth, those tiles run as 2, 4 or 8 workgroups each over parts of
- * their key chunks, and a merge kernel combines the parts (same masks,
- * rounding points and outputs).  Bytes needed
+ * tiles fill at most half of the GPU and visit more than a chunk or two each,
+ * or the last of several rounds of them fills at most a fifth, those tiles run
+ * as 2, 4 or 8 workgroups each over parts of their key chunks, and a merge
+ * kernel combines the parts (same masks, rounding points and outputs).  Bytes needed
  * from srswa_gather_fwd_workspace (0: no split for this shape); ws NULL or
  * short runs every tile whole.  The same reference kernels as
  * srswa_gather_fwd (HF/sparse_gather_triton.py:35-122,
@@ -219,7 +219,8 @@ typedef struct {
 
 int srswa_gather_fwd_paged(const srswa_paged_fwd_args* a, void* stream);
 
-/* srswa_gather_fwd_paged with a workspace: a launch of few tiles runs each as
+/* srswa_gather_fwd_paged with a workspace: a launch of few tiles (those past a
+ * request's rows counted) that visit more than a chunk or two each runs each as
  * several workgroups over parts of its key chunks, and a merge kernel combines
  * the parts (same masks, rounding points and outputs).  Bytes needed from
  * srswa_gather_fwd_paged_workspace (0: no split for this shape); ws NULL or

@@ -79,7 +79,11 @@ __device__ __forceinline__ float route_x(const srswa_dash_route_train_args& a, f
 // t, so Newton's steps from t = -1, left of the root (the largest z is 0),
 // stay left of it and reach it in a few; the closed form over the z above the
 // last t then gives tau in fp64.  t ends within 1e-6 of the root: a z that
-// close to it on the wrong side changes the closed form by its square.
+// close to it on the wrong side changes the closed form by its square.  Over 400
+// rows of 16 to 8,192 values, clusters at the root among them, tau was within
+// 5e-12 of the root in 80 bits; the sorted form, its support decided by fp64
+// prefix sums, within 4e-11, the closed form's own rounding.  (Newton's steps in
+// fp64: 55 us instead of 35, 41 instead of 29.)
 template <typename Each>
 __device__ __forceinline__ double entmax_threshold(Each&& each_z) {
   float t = -1.f;

@@ -121,6 +121,9 @@ void fwd_kernel(FwdK p) {
   // (runs of 2, 4 and 8 tiles per XCD: 169 and 143 us).  A single request has
   // no other length to balance and keeps the eighths, whole tiles of it at least:
   // 4,000 rows 89.6 us against 91.5 in turn, 16,000 rows 258 against 272.
+  // Requests x heads a multiple of 8: a (request, head) keeps to one XCD, and one
+  // long request among seven of 100 rows fills it to 1.5 (ten heads) or 3.4 (two)
+  // times the mean of live tiles, by count; in eighths to 6.6 times.
   const int nwhole = p.nlogical - p.ntail;
   int lid, part = 0, rec = -1;
   if constexpr (PAGED) {
