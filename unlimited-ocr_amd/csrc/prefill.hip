@@ -1038,7 +1038,10 @@ int plan_fwd_paged(const srswa_paged_fwd_args* a, FwdK& k, size_t& smem, size_t&
   const int umax = (int)std::min<int64_t>(nchunk, per_tile);
   const size_t setup = (3 * 64 + 4) * 4 + (size_t)k.nwords * 4;
   const int cus = device_cu_count();
-  // LDS of the layout with `tile` bytes of K and V, and the workgroups a CU holds with it
+  // LDS of the layout with `tile` bytes of K and V, and the workgroups a CU holds
+  // with it: by registers two waves per SIMD at D = 128 and three at D = 64; the
+  // LDS is given out in units of 1,280 bytes
+  const int held = a->D == 128 ? 4 : 6;
   auto layout = [&](size_t tile) {
     size_t n = std::max(tile, setup);
     k.chunks_off = (int)n;
@@ -1053,7 +1056,7 @@ int plan_fwd_paged(const srswa_paged_fwd_args* a, FwdK& k, size_t& smem, size_t&
     k.page_cap = (int)std::min<int64_t>(umax, k.pages_off < (int)budget ? (budget - k.pages_off) / (4 * k.ppc) : 0);
     n = k.pages_off + (size_t)k.page_cap * 4 * k.ppc;
     smem = (n + 15) / 16 * 16;
-    return std::min<int>(4, (int)((160 * 1024) / smem));
+    return std::min<int>(held, (int)((160 * 1024) / ((smem + 1279) / 1280 * 1280)));
   };
   // The V pitch without conflicts, unless the launch needs more rounds with it
   // than with the shorter one, or runs in fewer parts.  Ten heads, biased rows of
@@ -1062,7 +1065,9 @@ int plan_fwd_paged(const srswa_paged_fwd_args* a, FwdK& k, size_t& smem, size_t&
   // of 2,048 rows after 30,000 keys 181 -> 164; one of 2,560 rows (whole -> two
   // parts) 85 -> 69, of 1,472 (two -> four) 57 -> 50.  The same workgroups per CU
   // either way: 2,048 rows after 62,000 keys 182 -> 184, twelve slots 245 -> 247;
-  // one round, whole either way: 4,000 rows 90.8 -> 91.5.
+  // one round, whole either way: 4,000 rows 90.8 -> 91.5.  At D = 64 both pitches
+  take the same time and only the workgroups count: seven requests of 1 to 1,425
+  rows, sixteen heads, twelve slots, 2,576 tiles, five or six to a CU: 168 -> 122.
   const size_t wide = a->D == 128 ? FwdLds<128>::tileBytes : FwdLds<64>::tileBytes;
   const size_t narrow = a->D == 128 ? FwdLds<128, 2, true>::tileBytes : FwdLds<64, 2, true>::tileBytes;
   // Every tile is split or none: which tiles are live is known on the device
@@ -1071,11 +1076,11 @@ int plan_fwd_paged(const srswa_paged_fwd_args* a, FwdK& k, size_t& smem, size_t&
   // many short requests that would leave CUs idle may run whole).
   auto parts = [&](int per_cu) {
     if (cus <= 0 || per_cu <= 0) return 1;
-    return split_parts(nlogical, (int64_t)cus * per_cu, cus, mean_chunks2(nchunk, k.ntiles, umax), false, true);
+    return split_parts(nlogical, (int64_t)cus * std::min(per_cu, 4), cus, mean_chunks2(nchunk, k.ntiles, umax), false, true);
   };
   int per_cu = layout(wide);
   const bool fits = smem <= 156 * 1024;
-  if (!fits || per_cu < 4) {
+  if (!fits || per_cu < held) {
     const int with_narrow = layout(narrow);
     k.narrow = !fits || (with_narrow > per_cu &&
                          (nlogical > (int64_t)cus * per_cu || parts(with_narrow) > parts(per_cu)));
