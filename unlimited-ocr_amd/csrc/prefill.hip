@@ -1066,8 +1066,8 @@ int plan_fwd_paged(const srswa_paged_fwd_args* a, FwdK& k, size_t& smem, size_t&
   // parts) 85 -> 69, of 1,472 (two -> four) 57 -> 50.  The same workgroups per CU
   // either way: 2,048 rows after 62,000 keys 182 -> 184, twelve slots 245 -> 247;
   // one round, whole either way: 4,000 rows 90.8 -> 91.5.  At D = 64 both pitches
-  take the same time and only the workgroups count: seven requests of 1 to 1,425
-  rows, sixteen heads, twelve slots, 2,576 tiles, five or six to a CU: 168 -> 122.
+  // take the same time and only the workgroups count: seven requests of 1 to 1,425
+  // rows, sixteen heads, twelve slots, 2,576 tiles, five or six to a CU: 168 -> 122.
   const size_t wide = a->D == 128 ? FwdLds<128>::tileBytes : FwdLds<64>::tileBytes;
   const size_t narrow = a->D == 128 ? FwdLds<128, 2, true>::tileBytes : FwdLds<64, 2, true>::tileBytes;
   // Every tile is split or none: which tiles are live is known on the device
