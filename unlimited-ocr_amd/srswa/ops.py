@@ -68,6 +68,7 @@ def prepare_gather_decode(q, k_cache, v_cache, block_indices, q_pos, *, block_si
         if q_pos.dim() == 1:
             q_pos = q_pos.unsqueeze(1)
     B, Lq, HQ, D = q.shape
+    dev = q.device
     Bk, L, HKV, Dk = k_cache.shape
     if Bk != B or Dk != D or v_cache.shape != k_cache.shape:
         raise ValueError(f"cache shape {tuple(k_cache.shape)} / {tuple(v_cache.shape)} vs q {tuple(q.shape)}")
@@ -76,9 +77,9 @@ def prepare_gather_decode(q, k_cache, v_cache, block_indices, q_pos, *, block_si
         raise ValueError(f"block_indices shape {tuple(block_indices.shape)} != {(B, HI, Lq, S)}")
     if q.dtype != k_cache.dtype or q.dtype != v_cache.dtype:
         raise ValueError("q, k_cache, v_cache must share a dtype")
-    for t in (q, k_cache, v_cache):
-        if t.stride(-1) != 1:
-            raise UnsupportedShape("head dim must be contiguous")
+    qs, ks, vs = q.stride(), k_cache.stride(), v_cache.stride()
+    if qs[3] != 1 or ks[3] != 1 or vs[3] != 1:
+        raise UnsupportedShape("head dim must be contiguous")
     idx = _i32(block_indices).contiguous()
     if bias is not None:
         bias = _as(bias, torch.float32, idx.shape)
@@ -90,15 +91,15 @@ def prepare_gather_decode(q, k_cache, v_cache, block_indices, q_pos, *, block_si
     kvl = None if kv_len is None else _i32(kv_len).contiguous()
     odt = out_dtype or q.dtype
     if out is None:
-        out = torch.empty(B, Lq, HQ, D, dtype=odt, device=q.device)
+        out = torch.empty(B, Lq, HQ, D, dtype=odt, device=dev)
     elif squeeze:
         out = out.unsqueeze(1)
-    lse = torch.empty(B, Lq, HQ, dtype=torch.float32, device=q.device) if return_lse else None
+    lse = torch.empty(B, Lq, HQ, dtype=torch.float32, device=dev) if return_lse else None
 
     a = _lib.DecodeArgs()
-    a.q = q.data_ptr(); a.q_sb, a.q_sq, a.q_sh = q.stride()[:3]
-    a.k = k_cache.data_ptr(); a.k_sb, a.k_st, a.k_sh = k_cache.stride()[:3]
-    a.v = v_cache.data_ptr(); a.v_sb, a.v_st, a.v_sh = v_cache.stride()[:3]
+    a.q = q.data_ptr(); a.q_sb, a.q_sq, a.q_sh = qs[:3]
+    a.k = k_cache.data_ptr(); a.k_sb, a.k_st, a.k_sh = ks[:3]
+    a.v = v_cache.data_ptr(); a.v_sb, a.v_st, a.v_sh = vs[:3]
     a.idx = idx.data_ptr()
     a.idx_sb, a.idx_sh, a.idx_sq, a.idx_ss = idx.stride()[:4]
     a.bias = _lib.ptr(bias)
@@ -115,10 +116,10 @@ def prepare_gather_decode(q, k_cache, v_cache, block_indices, q_pos, *, block_si
     a.out_dtype = _lib.dtype_code(odt)
     L_ = _lib.lib()
     nscr = L_.srswa_gather_decode_workspace(ctypes.byref(a))
-    scr = _lib.scratch(q.device, nscr)
+    scr = _lib.scratch(dev, nscr)
     launch = _Launch(L_.srswa_gather_decode, a,
                      (q, k_cache, v_cache, idx, bias, valid, pos, kvl, out, lse),
-                     (scr, nscr), _lib.stream_ptr(q.device), "srswa_gather_decode")
+                     (scr, nscr), _lib.stream_ptr(dev), "srswa_gather_decode")
     if squeeze:
         out = out.squeeze(1)
         if lse is not None:
@@ -193,15 +194,16 @@ def prepare_index_meanpool_topk(q, k, q_pos, *, block_size, local_blocks, topk, 
     if k.stride(-1) != 1:
         raise UnsupportedShape("key head dim must be contiguous")
     nblk = int(nblk) if nblk is not None else -(-L // int(block_size))
-    qf = q.to(torch.float32)
+    dev = q.device
+    qf = q if q.dtype == torch.float32 else q.to(torch.float32)
     pos = _i32(q_pos).contiguous()
     if pos.shape != (B, Lq):
         raise ValueError(f"q_pos shape {tuple(pos.shape)} != {(B, Lq)}")
     kvl = None if kv_len is None else _i32(kv_len).contiguous()
     hc = None if head_cls is None else head_cls.to(torch.float32).contiguous()
-    scores = torch.empty(B, HI, Lq, nblk, dtype=torch.float32, device=q.device) if return_scores else None
-    kbar = torch.empty(B, HI, nblk, D, dtype=torch.float32, device=q.device) if return_kbar else None
-    idx = torch.empty(B, HI, Lq, int(topk), dtype=torch.int32, device=q.device) if topk > 0 else None
+    scores = torch.empty(B, HI, Lq, nblk, dtype=torch.float32, device=dev) if return_scores else None
+    kbar = torch.empty(B, HI, nblk, D, dtype=torch.float32, device=dev) if return_kbar else None
+    idx = torch.empty(B, HI, Lq, int(topk), dtype=torch.int32, device=dev) if topk > 0 else None
 
     a = _lib.IndexArgs()
     a.q = qf.data_ptr(); a.q_sb, a.q_sh, a.q_sq = qf.stride()[:3]
@@ -221,9 +223,9 @@ def prepare_index_meanpool_topk(q, k, q_pos, *, block_size, local_blocks, topk, 
     a.k_dtype = _lib.dtype_code(k.dtype)
     L_ = _lib.lib()
     nscr = L_.srswa_index_workspace(ctypes.byref(a))
-    scr = _lib.scratch(q.device, nscr)
+    scr = _lib.scratch(dev, nscr)
     launch = _Launch(L_.srswa_index_meanpool_topk, a, (qf, k, pos, kvl, hc, scores, kbar, idx),
-                     (scr, nscr), _lib.stream_ptr(q.device), "srswa_index_meanpool_topk")
+                     (scr, nscr), _lib.stream_ptr(dev), "srswa_index_meanpool_topk")
     if squeeze:
         idx = None if idx is None else idx.squeeze(2)
         scores = None if scores is None else scores.squeeze(2)
